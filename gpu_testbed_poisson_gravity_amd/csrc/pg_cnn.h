@@ -32,13 +32,14 @@ hipError_t cnn_mse(const float* D, const float* T, float* dY, float* partial, in
 // Adds the residual term of the loss (weight w) to dY and to the nblocks loss partials cnn_mse wrote.
 hipError_t cnn_res_loss(const float* D, const float* T, float* dY, float* partial, int n, float w, int nblocks,
                         hipStream_t s);
-hipError_t cnn_relu_bwd(const float* dY, const uint16_t* H, uint16_t* dH, float* bpart, size_t count, int nblocks,
-                        hipStream_t s);
+hipError_t cnn_relu_bwd(const float* dY, const uint16_t* H, uint16_t* dH, size_t count, int nblocks, hipStream_t s);
 hipError_t cnn_conv_bwd_data(const uint16_t* dH, const uint16_t* WT, const float* dYres, float* dX, int n,
                              hipStream_t s);
-int cnn_bwd_weight_blocks(int n);
-hipError_t cnn_conv_bwd_weight(const uint16_t* X, const uint16_t* dH, float* wpart, int n, hipStream_t s);
-hipError_t cnn_reduce_parts(const float* part, int parts, int len, float* dst, hipStream_t s);
+// Weight and bias gradients of all layers from their inputs x [n][10^3][16] (x[0]: the packed input, x[l]: y_l) and
+// output gradients dH [6][n][8^3][16], into g (parameter order).  part: [6][cnn_grad_parts(n)][kCnnLayerParams] floats.
+int cnn_grad_parts(int n);
+hipError_t cnn_weight_grad(const uint16_t* const (&x)[kCnnLayers], const uint16_t* dH, int n, float* part, float* g,
+                           hipStream_t s);
 hipError_t cnn_adam(float* p, const float* g, float* m, float* v, int n, float lr, float b1, float b2, float eps,
                     float c1, float c2, hipStream_t s);
 // Wb: [6][16][kCnnKF] forward layout; WT: [6][16][432] per-tap transposed (input-gradient pass); WL: the forward

@@ -257,26 +257,11 @@ __global__ void __launch_bounds__(kThreads) res_loss_kernel(const float* __restr
   if (threadIdx.x == 0) partial[blockIdx.x] += w * red[0];
 }
 
-// dH = dY * (H > 0) (or dY when H is null: the linear output layer), stored BF16 for the matrix cores;
-// per-block partial bias gradients (thread t always handles channel t % 16).
+// dH = dY * (H > 0) (or dY when H is null: the linear output layer), stored BF16 for the matrix cores.
 __global__ void __launch_bounds__(kThreads) relu_bwd_kernel(const float* __restrict__ dY, const u16* __restrict__ H,
-                                                            u16* __restrict__ dH, float* __restrict__ bpart,
-                                                            size_t count) {
-  __shared__ float red[kThreads];
-  float s = 0.0f;
-  for (size_t i = (size_t)blockIdx.x * kThreads + threadIdx.x; i < count; i += (size_t)gridDim.x * kThreads) {
-    const float g = (H == nullptr || bf2f(H[i]) > 0.0f) ? dY[i] : 0.0f;
-    const u16 gb = f2bf(g);
-    dH[i] = gb;
-    s += bf2f(gb);
-  }
-  red[threadIdx.x] = s;
-  __syncthreads();
-  for (int o = kThreads / 2; o >= CH; o >>= 1) {
-    if ((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-    __syncthreads();
-  }
-  if (threadIdx.x < CH) bpart[(size_t)blockIdx.x * CH + threadIdx.x] = red[threadIdx.x];
+                                                            u16* __restrict__ dH, size_t count) {
+  for (size_t i = (size_t)blockIdx.x * kThreads + threadIdx.x; i < count; i += (size_t)gridDim.x * kThreads)
+    dH[i] = f2bf((H == nullptr || bf2f(H[i]) > 0.0f) ? dY[i] : 0.0f);
 }
 
 // Input gradient on the interior of the padded input: dX[p][ci] = sum_{tap,co} W[co][tap][ci] dH[p+1-tap][co]
@@ -333,70 +318,154 @@ __global__ void __launch_bounds__(kThreads) conv_bwd_data_kernel(const u16* __re
   }
 }
 
-// Weight gradient: dW[co][tap*16+ci] = sum_{n,v} dH[n][v][co] X[n][v+tap][ci], one partial per workgroup.
-// GEMM with M = 16 output channels, N = 432, K = voxels (32 per MFMA); operands gathered from LDS.
-__global__ void __launch_bounds__(kThreads) conv_bwd_weight_kernel(const u16* __restrict__ X, const u16* __restrict__ dH,
-                                                                   float* __restrict__ wpart) {
-  constexpr int xvec = (kTZ + 2) * kPlane / 8;
-  constexpr int hvec = kTZ * So * So * 2;
-  __shared__ uint4 smem[xvec + hvec];
-  const int n = blockIdx.x / kSlabs, z0 = (blockIdx.x % kSlabs) * kTZ;
-  const u16* xs = reinterpret_cast<const u16*>(smem);
-  const u16* hs = reinterpret_cast<const u16*>(smem + xvec);
-  const uint4* xsrc = reinterpret_cast<const uint4*>(X + ((size_t)n * S + z0) * kPlane);
-  for (int i = threadIdx.x; i < xvec; i += kThreads) smem[i] = xsrc[i];
-  const uint4* hsrc = reinterpret_cast<const uint4*>(dH + (((size_t)n * So + z0) * So * So) * CH);
-  for (int i = threadIdx.x; i < hvec; i += kThreads) smem[xvec + i] = hsrc[i];
-  __syncthreads();
-  constexpr int NT = K / 16;                  // 27 column tiles
-  constexpr int TPW = (NT + 3) / 4;           // tiles per wave
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  floatx4 acc[TPW];
+// Weight and bias gradients of all six layers, one launch: dW[co][tap*16+ci] = sum_{n,v} dH[n][v][co] X[n][v+tap][ci]
+// and db[co] = sum_{n,v} dH[n][v][co].  Block (b, l) sums the samples b, b + gridDim.x, ... of layer l + 1 in its
+// accumulators and writes one partial in the parameter layout of a layer (W [16][432], b [16]).
+//
+// GEMM with rows co, columns ci and K = voxels, one 16x16 tile per tap.  Both operands need 8 consecutive voxels of
+// one channel per lane, so a sample is staged transposed, [z][y][channel][8 x] (row pitch 272 B: the transposing
+// writes of 8 rows then fall on different banks, and a wave's operand read is four contiguous 256 B pieces).  A tap's
+// x shift is applied to the dH row in registers (voxels shifted out of the row meet the zero x border of X), so one
+// X operand serves three taps: per 32 voxels a wave reads 4 operands for its 9 tiles (wave = dz).  A tenth tile with
+// a column of ones is the bias gradient.
+// Layer 1's input may hold any values in its border (the caller's array): its y and z border rows are staged like the
+// others and the two x border columns are added by two extra K steps gathered from memory.
+// Bound by staging (LDS writes, L2 reads).  MI355X, 256 samples: 12.2 us per layer and, with one partial per half
+// sample summed by a serial loop, 1.06 ms per layer for the sums; now see grad_reduce_kernel.
+constexpr int kWThreads = 192;     // three waves, one per dz
+constexpr int kTRow = 136;         // u16 per staged row: 16 channels x 8 voxels and 8 of padding
+constexpr int kXRows = S * S, kHRows = So * So;
+
+// Two voxels' 8 channels (h: channel half) into a staged row, as (voxel, voxel + 1) pairs per channel.
+__device__ __forceinline__ void stage_pair(u16* row, int xp, int h, const uint4& v0, const uint4& v1) {
+  const uint32_t a[4] = {v0.x, v0.y, v0.z, v0.w}, b[4] = {v1.x, v1.y, v1.z, v1.w};
+  uint32_t* d = reinterpret_cast<uint32_t*>(row + 64 * h) + xp;
 #pragma unroll
-  for (int i = 0; i < TPW; i++) acc[i] = floatx4{0.f, 0.f, 0.f, 0.f};
-  constexpr int M = kTZ * So * So;            // 128 voxels = 4 K steps
-  const int kq = 8 * (lane >> 4);
-  for (int k0 = 0; k0 < M; k0 += 32) {
-    // A[i = co][k = voxel]: dH[v][co] for the lane's 8 voxels
-    Pack8 a;
-#pragma unroll
-    for (int e = 0; e < 8; e++) a.h[e] = hs[(k0 + kq + e) * CH + (lane & 15)];
-#pragma unroll
-    for (int i = 0; i < TPW; i++) {
-      const int tile = wave * TPW + i;
-      if (tile >= NT) break;
-      const int col = tile * 16 + (lane & 15);
-      const int tap = col / CH, ci = col % CH;
-      const int dz = tap / 9, dy = (tap / 3) % 3, dx = tap % 3;
-      Pack8 b;
-#pragma unroll
-      for (int e = 0; e < 8; e++) {
-        const int v = k0 + kq + e;
-        const int lz = v / (So * So), oy = (v / So) % So, ox = v % So;
-        b.h[e] = xs[(((lz + dz) * S + oy + dy) * S + ox + dx) * CH + ci];
-      }
-      acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.v, b.v, acc[i], 0, 0, 0);
-    }
-  }
-  // D[i = co][j = col]: lane holds col = tile*16 + lane%16, co = 4*(lane/16) + r
-  float* out = wpart + (size_t)blockIdx.x * 16 * K;
-#pragma unroll
-  for (int i = 0; i < TPW; i++) {
-    const int tile = wave * TPW + i;
-    if (tile >= NT) break;
-    const int col = tile * 16 + (lane & 15);
-#pragma unroll
-    for (int r = 0; r < 4; r++) out[(4 * (lane >> 4) + r) * K + col] = acc[i][r];
+  for (int j = 0; j < 4; j++) {
+    d[8 * j] = (a[j] & 0xffffu) | (b[j] << 16);
+    d[8 * j + 4] = (a[j] >> 16) | (b[j] & 0xffff0000u);
   }
 }
 
-// Sum `parts` partial vectors of length len (fixed order: deterministic) and store into dst.
-__global__ void reduce_parts_kernel(const float* __restrict__ part, int parts, int len, float* __restrict__ dst) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= len) return;
+struct GradInputs {
+  const u16* x[kCnnLayers];   // input of each layer, padded [n][10^3][16]
+};
+
+template <bool BORDER>
+__device__ __forceinline__ void weight_grad_block(const u16* __restrict__ X, const u16* __restrict__ dH, int n,
+                                                  float* __restrict__ out, u16* xs, u16* hs) {
+  const int lane = threadIdx.x & 63, dz = threadIdx.x >> 6, g = lane >> 4, c = lane & 15;
+  if (!BORDER)   // the zero y and z border of the activations
+    for (int i = threadIdx.x; i < kXRows * kTRow / 8; i += kWThreads) {
+      const int r = i / (kTRow / 8), y = r % S, z = r / S;
+      if (y == 0 || y == S - 1 || z == 0 || z == S - 1) reinterpret_cast<uint4*>(xs)[i] = make_uint4(0, 0, 0, 0);
+    }
+  floatx4 acc[9], accb = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int t = 0; t < 9; t++) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+  Pack8 one;
+  one.u = make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u);
+  for (int smp = blockIdx.x; smp < n; smp += gridDim.x) {
+    const uint4* xg = reinterpret_cast<const uint4*>(X + (size_t)smp * kCnnInput);
+    const uint4* hg = reinterpret_cast<const uint4*>(dH + (size_t)smp * kCnnVox * CH);
+    constexpr int XR = BORDER ? kXRows : kHRows;
+    for (int i = threadIdx.x; i < XR * 8; i += kWThreads) {
+      const int r = i >> 3, xp = i & 3, h = (i >> 2) & 1;
+      const int z = BORDER ? r / S : r / So + 1, y = BORDER ? r % S : r % So + 1;
+      const uint4* s = xg + ((z * S + y) * S + 2 * xp + 1) * 2 + h;
+      stage_pair(xs + (z * S + y) * kTRow, xp, h, s[0], s[2]);
+    }
+    for (int i = threadIdx.x; i < kHRows * 8; i += kWThreads) {
+      const int r = i >> 3, xp = i & 3, h = (i >> 2) & 1;
+      const uint4* s = hg + (r * So + 2 * xp) * 2 + h;
+      stage_pair(hs + r * kTRow, xp, h, s[0], s[2]);
+    }
+    __syncthreads();
+#pragma unroll 2
+    for (int ks = 0; ks < kHRows / 4; ks++) {
+      const int z = ks >> 1, y = 4 * (ks & 1) + g;
+      Pack8 a[3], b;
+      a[1].u = *reinterpret_cast<const uint4*>(hs + (z * So + y) * kTRow + 8 * c);
+      const uint4 d = a[1].u;
+      const uint32_t s01 = __builtin_amdgcn_alignbit(d.y, d.x, 16), s12 = __builtin_amdgcn_alignbit(d.z, d.y, 16),
+                     s23 = __builtin_amdgcn_alignbit(d.w, d.z, 16);
+      a[0].u = make_uint4(s01, s12, s23, d.w >> 16);   // dx = 0: input voxel x meets output voxel x + 1
+      a[2].u = make_uint4(d.x << 16, s01, s12, s23);   // dx = 2: output voxel x - 1
+#pragma unroll
+      for (int dy = 0; dy < 3; dy++) {
+        b.u = *reinterpret_cast<const uint4*>(xs + ((z + dz) * S + y + dy) * kTRow + 8 * c);
+#pragma unroll
+        for (int dx = 0; dx < 3; dx++)
+          acc[3 * dy + dx] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[dx].v, b.v, acc[3 * dy + dx], 0, 0, 0);
+      }
+      if (dz == 0) accb = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[1].v, one.v, accb, 0, 0, 0);
+    }
+    if (BORDER) {   // x = 0 meets output voxel 0 at dx = 0, x = 9 output voxel 7 at dx = 2; K = 32 (z, y) rows
+      const u16* xb = X + (size_t)smp * kCnnInput;
+      for (int ks = 0; ks < 2; ks++)
+#pragma unroll
+        for (int side = 0; side < 2; side++) {
+          const int z = 4 * ks + g;
+          Pack8 a, b;
+#pragma unroll
+          for (int e = 0; e < 8; e++) a.h[e] = hs[(z * So + e) * kTRow + 8 * c + 7 * side];
+#pragma unroll
+          for (int dy = 0; dy < 3; dy++) {
+#pragma unroll
+            for (int e = 0; e < 8; e++) b.h[e] = xb[(((z + dz) * S + e + dy) * S + 9 * side) * CH + c];
+            acc[3 * dy + 2 * side] =
+                __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.v, b.v, acc[3 * dy + 2 * side], 0, 0, 0);
+          }
+        }
+    }
+    __syncthreads();
+  }
+  // D[i = co][j = ci]: lane holds ci = lane%16, co = 4*(lane/16) + r
+#pragma unroll
+  for (int t = 0; t < 9; t++)
+#pragma unroll
+    for (int r = 0; r < 4; r++) out[(4 * g + r) * K + (9 * dz + t) * CH + c] = acc[t][r];
+  if (dz == 0 && c == 0) {
+#pragma unroll
+    for (int r = 0; r < 4; r++) out[CH * K + 4 * g + r] = accb[r];
+  }
+}
+
+__global__ void __launch_bounds__(kWThreads) weight_grad_kernel(GradInputs in, const u16* __restrict__ dH, int n,
+                                                                float* __restrict__ part) {
+  __shared__ __align__(16) u16 xs[kXRows * kTRow];
+  __shared__ __align__(16) u16 hs[kHRows * kTRow];
+  const int l = blockIdx.y;
+  const u16* h = dH + (size_t)l * n * kCnnVox * CH;
+  float* out = part + ((size_t)l * gridDim.x + blockIdx.x) * kCnnLayerParams;
+  if (l == 0)
+    weight_grad_block<true>(in.x[0], h, n, out, xs, hs);
+  else
+    weight_grad_block<false>(in.x[l], h, n, out, xs, hs);
+}
+
+// Sum of the partials of every layer ([6][parts][kCnnLayerParams]) into the gradient vector, in a fixed order: 16
+// threads per column, each over every 16th partial, then a tree.  Reads at most 6 * 128 partials (21 MB); one wave of
+// serial loops over 1024 (weights) and 4096 (biases) partials took 4.7 of the 5.15 ms of a 256-sample step.
+constexpr int kRCols = 16, kRGroups = 16;
+__global__ void __launch_bounds__(kRCols * kRGroups) grad_reduce_kernel(const float* __restrict__ part, int parts,
+                                                                        float* __restrict__ g) {
+  __shared__ float red[kRGroups][kRCols];
+  const int c = threadIdx.x % kRCols, q = threadIdx.x / kRCols;
+  const int col = blockIdx.x * kRCols + c, l = col / kCnnLayerParams;
+  static_assert(kCnnLayerParams % kRCols == 0, "whole blocks per layer");
+  const float* p = part + (size_t)l * parts * kCnnLayerParams + col % kCnnLayerParams;
   float s = 0.0f;
-  for (int p = 0; p < parts; p++) s += part[(size_t)p * len + i];
-  dst[i] = s;
+#pragma unroll 4
+  for (int i = q; i < parts; i += kRGroups) s += p[(size_t)i * kCnnLayerParams];
+  red[q][c] = s;
+  __syncthreads();
+#pragma unroll
+  for (int o = kRGroups / 2; o > 0; o >>= 1) {
+    if (q < o) red[q][c] += red[q + o][c];
+    __syncthreads();
+  }
+  if (q == 0) g[col] = red[0][c];
 }
 
 // Adam on the FP32 master weights.
@@ -964,9 +1033,8 @@ hipError_t cnn_res_loss(const float* D, const float* T, float* dY, float* partia
   return hipGetLastError();
 }
 
-hipError_t cnn_relu_bwd(const float* dY, const uint16_t* H, uint16_t* dH, float* bpart, size_t count, int nblocks,
-                        hipStream_t s) {
-  hipLaunchKernelGGL(relu_bwd_kernel, dim3(nblocks), dim3(kThreads), 0, s, dY, H, dH, bpart, count);
+hipError_t cnn_relu_bwd(const float* dY, const uint16_t* H, uint16_t* dH, size_t count, int nblocks, hipStream_t s) {
+  hipLaunchKernelGGL(relu_bwd_kernel, dim3(nblocks), dim3(kThreads), 0, s, dY, H, dH, count);
   return hipGetLastError();
 }
 
@@ -976,15 +1044,16 @@ hipError_t cnn_conv_bwd_data(const uint16_t* dH, const uint16_t* WT, const float
   return hipGetLastError();
 }
 
-int cnn_bwd_weight_blocks(int n) { return n * kSlabs; }
+// One partial per block and layer: 6 * 128 blocks are three per CU.
+int cnn_grad_parts(int n) { return n < 128 ? n : 128; }
 
-hipError_t cnn_conv_bwd_weight(const uint16_t* X, const uint16_t* dH, float* wpart, int n, hipStream_t s) {
-  hipLaunchKernelGGL(conv_bwd_weight_kernel, dim3(n * kSlabs), dim3(kThreads), 0, s, X, dH, wpart);
-  return hipGetLastError();
-}
-
-hipError_t cnn_reduce_parts(const float* part, int parts, int len, float* dst, hipStream_t s) {
-  hipLaunchKernelGGL(reduce_parts_kernel, dim3((len + 255) / 256), dim3(256), 0, s, part, parts, len, dst);
+hipError_t cnn_weight_grad(const uint16_t* const (&x)[kCnnLayers], const uint16_t* dH, int n, float* part, float* g,
+                           hipStream_t s) {
+  GradInputs in;
+  for (int l = 0; l < kCnnLayers; l++) in.x[l] = x[l];
+  const int parts = cnn_grad_parts(n);
+  hipLaunchKernelGGL(weight_grad_kernel, dim3(parts, kCnnLayers), dim3(kWThreads), 0, s, in, dH, n, part);
+  hipLaunchKernelGGL(grad_reduce_kernel, dim3(kCnnParams / kRCols), dim3(kRCols * kRGroups), 0, s, part, parts, g);
   return hipGetLastError();
 }
 

@@ -48,9 +48,8 @@ struct pgamd_cnn {
   bool train_ws = false;
   uint16_t* y[6] = {};      // y1..y5, padded [n][10^3][16] with zero borders (y[0] unused: the input)
   uint16_t* h[6] = {};      // pre-activations h1..h5 [n][8^3][16] (training only)
-  uint16_t* dh = nullptr;   // [n][8^3][16]
+  uint16_t* dh = nullptr;   // output gradients of the six layers, [6][n][8^3][16]
   float *d = nullptr, *dy6 = nullptr, *dyA = nullptr, *dyB = nullptr, *part = nullptr, *lossp = nullptr;
-  size_t part_floats = 0;
   // pipelined warm-start solve: fork event and one event per chunk
   hipEvent_t ev[kMaxChunks + 1] = {};
 };
@@ -92,13 +91,11 @@ int ensure_ws(pgamd_cnn* n, int count, bool train) {
   }
   ok &= hipMalloc(&n->d, c * kCnnOutputs * 4) == hipSuccess;
   if (train) {
-    ok &= hipMalloc(&n->dh, act * 2) == hipSuccess;
+    ok &= hipMalloc(&n->dh, kCnnLayers * act * 2) == hipSuccess;
     ok &= hipMalloc(&n->dy6, act * 4) == hipSuccess;
     ok &= hipMalloc(&n->dyA, act * 4) == hipSuccess;
     ok &= hipMalloc(&n->dyB, act * 4) == hipSuccess;
-    const size_t pf = std::max((size_t)cnn_bwd_weight_blocks(count) * kW, (size_t)reduce_blocks(act) * kCnnChannels);
-    ok &= hipMalloc(&n->part, pf * 4) == hipSuccess;
-    n->part_floats = pf;
+    ok &= hipMalloc(&n->part, (size_t)kCnnLayers * cnn_grad_parts(count) * kCnnLayerParams * 4) == hipSuccess;
     ok &= hipMalloc(&n->lossp, kMseBlocks * 4) == hipSuccess;
   }
   if (!ok) {
@@ -139,24 +136,23 @@ int forward_backward(pgamd_cnn* n, const uint16_t* x0, const float* target, int 
   if (rc != PGAMD_OK) return rc;
   const size_t act = (size_t)count * kCnnVox * kCnnChannels;
   const int nb = reduce_blocks(act);
-  const int wblocks = cnn_bwd_weight_blocks(count);
   CK(cnn_mse(n->d, target, n->dy6, n->lossp, count * kCnnVox, kMseBlocks, s));
   if (n->res_weight > 0.0f) CK(cnn_res_loss(n->d, target, n->dy6, n->lossp, count, n->res_weight, kMseBlocks, s));
   const float* dy = n->dy6;
   float* bufs[2] = {n->dyA, n->dyB};
   int which = 0;
   for (int l = 6; l >= 1; l--) {
-    CK(cnn_relu_bwd(dy, l == 6 ? nullptr : n->h[l], n->dh, n->part, act, nb, s));
-    CK(cnn_reduce_parts(n->part, nb, kCnnChannels, n->g + ob(l), s));
-    CK(cnn_conv_bwd_weight(l == 1 ? x0 : n->y[l - 1], n->dh, n->part, count, s));
-    CK(cnn_reduce_parts(n->part, wblocks, kW, n->g + ow(l), s));
+    uint16_t* dh = n->dh + (size_t)(l - 1) * act;
+    CK(cnn_relu_bwd(dy, l == 6 ? nullptr : n->h[l], dh, act, nb, s));
     if (l > 1) {
       float* dx = bufs[which];
       which ^= 1;
-      CK(cnn_conv_bwd_data(n->dh, n->wt + (size_t)(l - 1) * kW, l == 6 ? nullptr : dy, dx, count, s));
+      CK(cnn_conv_bwd_data(dh, n->wt + (size_t)(l - 1) * kW, l == 6 ? nullptr : dy, dx, count, s));
       dy = dx;
     }
   }
+  const uint16_t* x[kCnnLayers] = {x0, n->y[1], n->y[2], n->y[3], n->y[4], n->y[5]};
+  CK(cnn_weight_grad(x, n->dh, count, n->part, n->g, s));
   return PGAMD_OK;
 }
 
