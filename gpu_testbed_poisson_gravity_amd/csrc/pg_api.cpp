@@ -409,6 +409,7 @@ int pgamd_set_layout(pgamd_context* c, int gs, int ppw, int pad) {
                 "per wavefront)", pad);
   c->layout.ppw[gs] = ppw;
   c->layout.pad[gs] = pad;
+  c->layout.fixed[gs] = true;
   return PGAMD_OK;
 }
 

@@ -72,6 +72,102 @@ __device__ __forceinline__ void interp_children(const T (&v)[3][3][3], int int_s
   }
 }
 
+// The same operations child by child, arranged for few registers: at(dk, dj, di) is the value at that offset (0..2) of the
+// 3^3 neighbourhood, and the eight sums advance together, a slope (or neighbour) at a time, so that little besides them is
+// live.  FENCE: keeps the compiler from loading the whole neighbourhood first.  The kernels that keep their cells in
+// registers during the interpolation use this form (FP64 block SOR, ghost size 5: 300 bytes of spills per lane with the
+// form above, none with this one); the compact one-wavefront SOR kernel allocates its 256 registers better with the form
+// above (1.00 against 1.22 ms for 16384 patches).
+template <bool FENCE, typename T, class At>
+__device__ __forceinline__ void interp_children_at(At at, int int_scheme, T (&ch)[2][2][2]) {
+  auto fence = [](int q) {
+    if (FENCE && q % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+  };
+  if (int_scheme == kIntCQuad) {
+    // slope q: scale, and the offsets of its two values; its sign in child (cz, cy, cx) is the product of the signs of the
+    // axes in `ax` (bit 0 x, 1 y, 2 z), negated where `neg`
+    constexpr struct {
+      float scale;
+      int p[3], m[3], ax;
+      bool neg;
+    } S[13] = {{0.125f, {1, 1, 2}, {1, 1, 0}, 1, false},       {0.125f, {1, 2, 1}, {1, 0, 1}, 2, false},
+               {0.125f, {2, 1, 1}, {0, 1, 1}, 4, false},       {0.015625f, {0, 1, 2}, {0, 1, 0}, 5, true},
+               {0.015625f, {0, 2, 1}, {0, 0, 1}, 6, true},     {0.015625f, {1, 0, 2}, {1, 0, 0}, 3, true},
+               {0.015625f, {1, 2, 2}, {1, 2, 0}, 3, false},    {0.015625f, {2, 1, 2}, {2, 1, 0}, 5, false},
+               {0.015625f, {2, 2, 1}, {2, 0, 1}, 6, false},    {0.001953125f, {0, 0, 2}, {0, 0, 0}, 7, false},
+               {0.001953125f, {0, 2, 2}, {0, 2, 0}, 7, true},  {0.001953125f, {2, 0, 2}, {2, 0, 0}, 7, true},
+               {0.001953125f, {2, 2, 2}, {2, 2, 0}, 7, false}};
+#pragma unroll
+    for (int q = 0; q < 13; q++) {
+      const T s = T(S[q].scale) * (at(S[q].p[0], S[q].p[1], S[q].p[2]) - at(S[q].m[0], S[q].m[1], S[q].m[2]));
+#pragma unroll
+      for (int e = 0; e < 8; e++) {
+        const int minus = ((S[q].ax & 1) && !(e & 1)) + ((S[q].ax & 2) && !(e & 2)) + ((S[q].ax & 4) && !(e & 4)) + S[q].neg;
+        T& a = ch[e >> 2][(e >> 1) & 1][e & 1];
+        if (q == 0)
+          a = minus & 1 ? -s : s;
+        else
+          a = minus & 1 ? a - s : a + s;
+      }
+      fence(q);
+    }
+    const T parent = at(1, 1, 1);
+#pragma unroll
+    for (int e = 0; e < 8; e++) ch[e >> 2][(e >> 1) & 1][e & 1] = ch[e >> 2][(e >> 1) & 1][e & 1] + parent;
+  } else {
+    const T Mp[3] = {T(-0.09375), T(0.9375), T(0.15625)};
+    const T Mm[3] = {T(0.15625), T(0.9375), T(-0.09375)};
+#pragma unroll
+    for (int e = 0; e < 8; e++) ch[e >> 2][(e >> 1) & 1][e & 1] = T(0);
+#pragma unroll
+    for (int q = 0; q < 27; q++) {
+      const int dk = q / 9, dj = q / 3 % 3, di = q % 3;
+      const T v = at(dk, dj, di);
+#pragma unroll
+      for (int e = 0; e < 8; e++) {
+        const T wz = e & 4 ? Mp[dk] : Mm[dk];
+        const T wy = e & 2 ? Mp[dj] : Mm[dj];
+        const T wx = e & 1 ? Mp[di] : Mm[di];
+        T& a = ch[e >> 2][(e >> 1) & 1][e & 1];
+        a = a + v * wz * wy * wx;
+      }
+      fence(q);
+    }
+  }
+}
+
+// Coarse cell q (1-based i, j, k of the NC^3 block that has children in the cube) of the interpolation
+// loop: every cell, or (SHELL) only the 2 NC^2 + 4 (NC-1)(NC-2) cells on the outer layer of the block, whose
+// children include every cell of the cube's Dirichlet layer (the only cells a zero start or a caller's guess
+// leaves to the interpolation).
+template <int NC, bool SHELL>
+__device__ __forceinline__ void coarse_cell(int q, int& i, int& j, int& k) {
+  if (!SHELL) {
+    i = q % NC + 1;
+    j = (q / NC) % NC + 1;
+    k = q / (NC * NC) + 1;
+    return;
+  }
+  constexpr int F = NC * NC, RING = 4 * (NC - 1);
+  if (q < 2 * F) {   // the bottom and top faces
+    const int t = q % F;
+    k = q < F ? 1 : NC;
+    i = t % NC + 1;
+    j = t / NC + 1;
+    return;
+  }
+  const int r = q - 2 * F, t = r % RING;   // the ring of each layer in between
+  k = r / RING + 2;
+  if (t < 2 * NC) {
+    j = t < NC ? 1 : NC;
+    i = t % NC + 1;
+  } else {
+    const int u = t - 2 * NC;
+    i = u < NC - 2 ? 1 : NC;
+    j = u % (NC - 2) + 2;
+  }
+}
+
 // Cell q of the outer layer of an N^3 cube (faces z = 0 and N-1, then the ring of each layer in between).
 template <int N>
 __device__ __forceinline__ void shell_cell(int q, int& x, int& y, int& z) {

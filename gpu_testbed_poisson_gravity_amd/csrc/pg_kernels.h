@@ -134,9 +134,10 @@ struct ParamsByGs {
   SolveParams p[6];
 };
 
-// Per-ghost-size launch layout of the SOR kernel: patches per wavefront.  Chosen by the autotuner;
+// Per-ghost-size launch layout of the one-wavefront SOR kernel: patches per wavefront.  Chosen by the autotuner;
 // the default is the densest packing that fits one wavefront.
 struct SorLayout {
+  bool fixed[6];           // set by the caller: always the one-wavefront kernel, never the block form
   int ppw[6];              // patches per wavefront, indexed by gs
   int pad[6];              // split-row padding in floats (bank-conflict avoidance), or kPadCompact, by gs
   int waves_per_cu;        // persistent kernel occupancy target
@@ -169,10 +170,18 @@ bool supported_layout(int gs, int ppw, int pad);
 size_t lds_bytes_sor(int gs, int ppw, int pad);
 size_t lds_bytes_mg(int gs);
 int supported_ppw(int gs, int ppw);
-// FP64 kernels (pg_f64.hip and the FP64 instances of the MG kernel): one workgroup per patch.
+// FP64 kernels (pg_f64.hip, and the FP64 instances of the block SOR and MG kernels): one workgroup per patch.
 hipError_t launch_uniform64(const UniformBatch64& b, const SolveParams64& p, hipStream_t stream);
 hipError_t launch_gravity64(const double* pot, double* flu, int npatch, int gra_ghost, double gra_const, int p5,
                             hipStream_t stream);
+// Block form of the SOR kernel, several wavefronts per patch.  FP32: same results and counts as the one-wavefront kernel;
+// wave_dpp is the order of its relative-residual sums (layouts with one patch per wavefront), ppw the patches per task of
+// a mixed batch.
+bool sor_blocks_better(int gs, int npatch);
+hipError_t launch_sor_blocks(const UniformBatch& b, const SolveParams& p, bool wave_dpp, hipStream_t s);
+hipError_t launch_sor_blocks_tasks(const MixedBatch& b, const SolveParams& p, int gs, int ppw, int first, int count,
+                                   hipStream_t s);
+hipError_t launch_sor_blocks64(const UniformBatch64& b, const SolveParams64& p, hipStream_t s);
 hipError_t launch_mg_uniform64(const UniformBatch64& b, const SolveParams64& p, hipStream_t s);
 
 }  // namespace pgamd

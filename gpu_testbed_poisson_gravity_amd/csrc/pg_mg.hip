@@ -21,6 +21,7 @@
 #include "pg_geometry.h"
 #include "pg_kernels.h"
 #include "pg_interp.h"
+#include "pg_reduce.h"
 
 #pragma clang fp contract(off)
 
@@ -129,7 +130,7 @@ struct MgGeo {
 };
 // Waves per SIMD mg_patch is compiled for: FP32 fits 4 in 128 registers and FP64 2 in 256; with two planes per thread one
 // more FP32 wave (not at ghost size 1, whose single wave does all the rest of a patch and would spill).
-constexpr int mg_waves(int gs, size_t word) { return word == 8 ? 2 : gs == 2 || gs == 4 ? 5 : 4; }
+constexpr int mg_waves(int gs, size_t word) { return (word == 8 ? 2 : 4) + (gs == 2 || gs == 4); }
 // workgroup of mg_patch_cells: one thread per cell of a colour
 constexpr int mg_cell_threads(int gs) { return gs == 1 ? 256 : 512; }
 constexpr int kMgMaxThreads = MgGeo<4>::THREADS;   // workgroup of the persistent kernel, enough for any ghost size
@@ -157,26 +158,6 @@ __device__ __forceinline__ void level_sync() {
   } else {
     __syncthreads();
   }
-}
-
-// v of the lane a DPP control selects (within a row of 16 lanes)
-template <int CTRL>
-__device__ __forceinline__ float dpp(float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, false));
-}
-template <int CTRL>
-__device__ __forceinline__ double dpp(double v) {
-  return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xF, 0xF, false),
-                          __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xF, 0xF, false));
-}
-// Sum over each row of 16 lanes, the same bits in every lane of the row: partners 1 and 2 apart, then the mirrored
-// halves of 8 and of 16 lanes.
-template <typename T>
-__device__ __forceinline__ T row_sum(T v) {
-  v = v + dpp<0xB1>(v);
-  v = v + dpp<0x4E>(v);
-  v = v + dpp<0x141>(v);
-  return v + dpp<0x140>(v);
 }
 
 // Block-wide sums of two values in a fixed order (bitwise reproducible for a given launch shape): rows of 16 lanes by
@@ -490,14 +471,8 @@ __device__ void mg_patch(T* __restrict__ lds, const T* __restrict__ rho, const T
   __syncthreads();
   constexpr int NC = C - 2, MX = M::MX;
   auto children = [&](int i, int j, int k, T (&ch)[2][2][2]) {
-    T v[3][3][3];
-#pragma unroll
-    for (int dk = 0; dk < 3; dk++)
-#pragma unroll
-      for (int dj = 0; dj < 3; dj++)
-#pragma unroll
-        for (int di = 0; di < 3; di++) v[dk][dj][di] = stage[((k + dk - 1) * C + (j + dj - 1)) * C + (i + di - 1)];
-    interp_children(v, P.int_scheme, ch);
+    const T* c = stage + ((k - 1) * C + j - 1) * C + i - 1;
+    interp_children_at<false>([&](int dk, int dj, int di) { return c[(dk * C + dj) * C + di]; }, P.int_scheme, ch);
   };
   if constexpr (U == 1) {
     // A thread's block is whole coarse cells: straight into registers.  The faces' coarse cells and, for a window that
@@ -784,10 +759,9 @@ __device__ void mg_patch_cells(T* __restrict__ lds, const T* __restrict__ rho, c
   __syncthreads();
   if (t < NC * NC * NC) {
     const int i = t % NC + 1, j = (t / NC) % NC + 1, k = t / (NC * NC) + 1;
-    T v[3][3][3], ch[2][2][2];
-#pragma unroll
-    for (int e = 0; e < 27; e++) v[e / 9][e / 3 % 3][e % 3] = stage[nat(C, i - 1 + e % 3, j - 1 + e / 3 % 3, k - 1 + e / 9)];
-    interp_children(v, P.int_scheme, ch);
+    T ch[2][2][2];
+    const T* c = stage + nat(C, i - 1, j - 1, k - 1);
+    interp_children_at<false>([&](int dk, int dj, int di) { return c[nat(C, di, dj, dk)]; }, P.int_scheme, ch);
 #pragma unroll
     for (int e = 0; e < 8; e++) {
       const int fx = 2 * (i - 1) + (e & 1) - U, fy = 2 * (j - 1) + ((e >> 1) & 1) - U, fz = 2 * (k - 1) + (e >> 2) - U;
@@ -886,12 +860,12 @@ __device__ void mg_patch_cells(T* __restrict__ lds, const T* __restrict__ rho, c
 }
 
 // How a batch is run: mg_patch, or for a small batch at ghost sizes 1 and 2 mg_patch_cells (see mg_small).
-enum MgForm { kMgBlocks, kMgCells, kMgPacked };   // kMgPacked: mg_patch with one more wave per SIMD, some spills
+enum MgForm { kMgBlocks, kMgCells };
 
 template <int GS, MgForm F, typename T>
 struct MgLaunch {
   static constexpr int THREADS = F == kMgCells ? mg_cell_threads(GS) : MgGeo<GS>::THREADS;
-  static constexpr int WAVES = F == kMgCells ? (sizeof(T) == 8 ? 2 : 4) : mg_waves(GS, sizeof(T)) + (F == kMgPacked);
+  static constexpr int WAVES = F == kMgCells ? (sizeof(T) == 8 ? 3 : 6) : mg_waves(GS, sizeof(T));
   static constexpr size_t LDS = sizeof(T) * (MgGeo<GS>::FLOATS + (F == kMgCells ? MgGeo<GS>::N * MgGeo<GS>::N * MgGeo<GS>::N : 0));
 };
 
@@ -954,9 +928,6 @@ template <int GS, typename PT>
 static hipError_t launch_mg(const UniformBatchT<typename PT::real>& b, const PT& p, hipStream_t s) {
   if constexpr (GS <= 2) {
     if (mg_small(GS, sizeof(typename PT::real), b.npatch)) return launch_mg_as<GS, kMgCells>(b, p, s);
-  }
-  if constexpr (GS == 2 && sizeof(typename PT::real) == 8) {
-    if (b.npatch > 1024) return launch_mg_as<GS, kMgPacked>(b, p, s);
   }
   return launch_mg_as<GS, kMgBlocks>(b, p, s);
 }

@@ -1,0 +1,48 @@
+// Wavefront sums shared by the SOR and MG kernels (device code).
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+namespace pgamd {
+
+// v of the lane a DPP control selects (within a row of 16 lanes)
+template <int CTRL>
+__device__ __forceinline__ float dpp(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, false));
+}
+template <int CTRL>
+__device__ __forceinline__ double dpp(double v) {
+  return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xF, 0xF, false),
+                          __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xF, 0xF, false));
+}
+
+// Sum over each row of 16 lanes, the same bits in every lane of the row: partners 1 and 2 apart in a quad, then the
+// mirrored halves of 8 and of 16 lanes (each step adds the same two operands in every lane of a pair, only commuted).
+template <typename T>
+__device__ __forceinline__ T row_sum(T v) {
+  v = v + dpp<0xB1>(v);    // quad [1,0,3,2]
+  v = v + dpp<0x4E>(v);    // quad [2,3,0,1]
+  v = v + dpp<0x141>(v);   // half-row mirror
+  return v + dpp<0x140>(v);   // row mirror
+}
+
+// Sum over the wavefront: rows of 16 lanes as above, then (r0 + r1) + (r2 + r3) from scalar registers, so every lane gets
+// the same bits.
+__device__ __forceinline__ float wave_sum_dpp(float v) {
+  v = row_sum(v);
+  const float r0 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 0));
+  const float r1 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 16));
+  const float r2 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 32));
+  const float r3 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 48));
+  return (r0 + r1) + (r2 + r3);
+}
+
+// Butterfly sum over the wavefront (partners 32, 16, ... 1 apart); with lanes beyond a shorter segment at zero, the bits
+// of the butterfly over that segment.
+__device__ __forceinline__ float wave_sum_butterfly(float v) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  return v;
+}
+
+}  // namespace pgamd

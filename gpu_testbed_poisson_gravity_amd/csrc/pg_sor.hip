@@ -30,6 +30,7 @@
 #include "pg_geometry.h"
 #include "pg_kernels.h"
 #include "pg_interp.h"
+#include "pg_reduce.h"
 #include "pg_internal.h"
 
 #pragma clang fp contract(off)
@@ -75,65 +76,21 @@ __device__ __forceinline__ float seg_sum(float v) {
   return v;
 }
 
-// Sum for the relative-residual test.  A whole wavefront (SEG = 64) reduces inside the VALU: DPP exchanges
-// within each row of 16 lanes (partners 1 and 2 apart in a quad, then the mirrored halves of 8 and of 16
-// lanes; each step adds the same two operands in every lane of a pair, only commuted), then the four row sums
-// read from lanes 0, 16, 32 and 48 are added as (r0 + r1) + (r2 + r3) from scalar registers, so every lane gets
-// the same bits.  seg_sum's butterfly crosses lanes through the LDS crossbar six times in a row; the stall
-// rule and the guess check keep that order.
+// Sum for the relative-residual test.  A whole wavefront (SEG = 64) reduces inside the VALU (wave_sum_dpp); seg_sum's
+// butterfly crosses lanes through the LDS crossbar six times in a row; the stall rule and the guess check keep that
+// order.
 template <int SEG>
 __device__ __forceinline__ float check_sum(float v) {
-  if constexpr (SEG != 64) {
+  if constexpr (SEG != 64)
     return seg_sum<SEG>(v);
-  } else {
-    v = v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xF, 0xF, false));  // quad [1,0,3,2]
-    v = v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xF, 0xF, false));  // quad [2,3,0,1]
-    v = v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xF, 0xF, false)); // half-row mirror
-    v = v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x140, 0xF, 0xF, false)); // row mirror
-    const float r0 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 0));
-    const float r1 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 16));
-    const float r2 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 32));
-    const float r3 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 48));
-    return (r0 + r1) + (r2 + r3);
-  }
+  else
+    return wave_sum_dpp(v);
 }
 
 // Any lane of the wavefront (a workgroup is exactly one wavefront here).
 __device__ __forceinline__ bool wave_any(bool pred) { return __ballot(pred) != 0; }
 
 // ---- interpolation into LDS --------------------------------------------------------------------------
-
-// Coarse cell q (1-based i, j, k of the NC^3 block that has children in the cube) of the interpolation
-// loop: every cell, or (SHELL) only the 2 NC^2 + 4 (NC-1)(NC-2) cells on the outer layer of the block, whose
-// children include every cell of the cube's Dirichlet layer (the only cells a zero start or a caller's guess
-// leaves to the interpolation).
-template <int NC, bool SHELL>
-__device__ __forceinline__ void coarse_cell(int q, int& i, int& j, int& k) {
-  if (!SHELL) {
-    i = q % NC + 1;
-    j = (q / NC) % NC + 1;
-    k = q / (NC * NC) + 1;
-    return;
-  }
-  constexpr int F = NC * NC, RING = 4 * (NC - 1);
-  if (q < 2 * F) {   // the bottom and top faces
-    const int t = q % F;
-    k = q < F ? 1 : NC;
-    i = t % NC + 1;
-    j = t / NC + 1;
-    return;
-  }
-  const int r = q - 2 * F, t = r % RING;   // the ring of each layer in between
-  k = r / RING + 2;
-  if (t < 2 * NC) {
-    j = t < NC ? 1 : NC;
-    i = t % NC + 1;
-  } else {
-    const int u = t - 2 * NC;
-    i = u < NC - 2 ? 1 : NC;
-    j = u % (NC - 2) + 2;
-  }
-}
 
 // Interpolate a patch's coarse potential into its LDS cube (split layout).  `lane`/`nlanes` index the
 // lanes serving this patch.  Two coarse cells per lane and step: both 27-value neighbourhoods are
@@ -1252,6 +1209,7 @@ int sor_uniform_blocks_per_cu(int gs, int ppw, int pad) {
 hipError_t launch_uniform(const UniformBatch& b, const SolveParams& p, const SorLayout& lay, hipStream_t s) {
   if (b.npatch <= 0) return hipSuccess;
   if (b.scheme == kSchemeMG) return launch_mg_uniform(b, p, s);
+  if (!lay.fixed[b.gs] && sor_blocks_better(b.gs, b.npatch)) return launch_sor_blocks(b, p, lay.ppw[b.gs] == 1, s);
   return launch_sor_uniform_dispatch(b, p, lay.ppw[b.gs], lay.pad[b.gs], s);
 }
 
