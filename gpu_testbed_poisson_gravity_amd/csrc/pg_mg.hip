@@ -12,7 +12,7 @@
 //
 // Bound: VALU issue and LDS reads, about evenly (GS 5, per patch and V-cycle of 3+3 sweeps: 9.4k wave VALU
 // instructions over 4 SIMDs and 8.9k LDS cycles).  The first form kept every cell and its right-hand side's index
-// arithmetic in 256 threads and read all seven operands from LDS.  MI355X, 4096 GS-5 patches: 551 -> 238 us.
+// arithmetic in 256 threads and read all seven operands from LDS.  MI355X, 4096 GS-5 patches: 551 -> 222 us.
 
 #include <hip/hip_runtime.h>
 
@@ -129,8 +129,10 @@ struct MgGeo {
   }
 };
 // Waves per SIMD mg_patch is compiled for: FP32 fits 4 in 128 registers and FP64 2 in 256; with two planes per thread one
-// more FP32 wave (not at ghost size 1, whose single wave does all the rest of a patch and would spill).
-constexpr int mg_waves(int gs, size_t word) { return (word == 8 ? 2 : 4) + (gs == 2 || gs == 4); }
+// more (not at ghost size 1, whose single wave does all the rest of a patch and would spill), and at ghost size 4 another
+// one: its workgroups of six waves then fit four to a CU instead of three (FP32 8192 patches 493 -> 452 us, FP64 2776 ->
+// 2051 us, for 28 bytes of spills that cost a lone patch 8%).
+constexpr int mg_waves(int gs, size_t word) { return (word == 8 ? 2 : 4) + (gs == 2 || gs == 4) + (gs == 4); }
 // workgroup of mg_patch_cells: one thread per cell of a colour
 constexpr int mg_cell_threads(int gs) { return gs == 1 ? 256 : 512; }
 constexpr int kMgMaxThreads = MgGeo<4>::THREADS;   // workgroup of the persistent kernel, enough for any ghost size
@@ -287,7 +289,8 @@ __device__ __forceinline__ T coarse_neighbours(const T* __restrict__ p) {
   return p[zs] + p[-zs] + p[ys] + p[-ys] + p[1] + p[-1];
 }
 
-template <int n, bool ONE_WAVE, typename T, int K>
+// FROM_ZERO: the solution is zero before the first sweep, whatever its interior holds: the first pass reads nothing.
+template <int n, bool ONE_WAVE, bool FROM_ZERO, typename T, int K>
 __device__ __forceinline__ void smooth_coarse(const MgCoarse<n>& k, T* __restrict__ sol, const T (&rhs)[K], T dh2, int times) {
   const T one_six = T(1) / T(6);
   const int odd = (k.x + k.y + k.z) & 1;                    // colour of the first cell
@@ -296,7 +299,11 @@ __device__ __forceinline__ void smooth_coarse(const MgCoarse<n>& k, T* __restric
   T *p1 = sol + k.id + x1, *p0 = sol + k.id + x0;
   const T q1 = dh2 * (x1 ? rhs[K - 1] : rhs[0]), q0 = dh2 * (x0 ? rhs[K - 1] : rhs[0]);
   for (int s = 0; s < times; s++) {
-    if (h1) *p1 = one_six * (coarse_neighbours<n>(p1) - q1);
+    if (FROM_ZERO && s == 0) {
+      if (h1) *p1 = one_six * (T(0) - q1);
+    } else {
+      if (h1) *p1 = one_six * (coarse_neighbours<n>(p1) - q1);
+    }
     level_sync<ONE_WAVE>();
     if (h0) *p0 = one_six * (coarse_neighbours<n>(p0) - q0);
     level_sync<ONE_WAVE>();
@@ -358,6 +365,34 @@ __device__ __forceinline__ T prolong_cell(const T* __restrict__ c0, const T (&wz
   return s;
 }
 
+// Correction of the thread's level-0 cells of one colour (ODD: colour 1) from level 1, published.
+template <bool ODD, int GS, typename T>
+__device__ __forceinline__ void prolongate_level0(MgOwned<GS, T>& o, T* __restrict__ lds) {
+  using M = MgGeo<GS>;
+  constexpr int n1 = M::n(1), N = M::N;
+  const T* cs = lds + M::off_sol(1);
+  T wx[2][2], wy[2][2];
+  int lx[2], ly[2];
+  const int x0 = opaque(o.x0), y0 = opaque(o.y0), z0 = opaque(o.z0);
+#pragma unroll
+  for (int u = 0; u < 2; u++) {
+    lx[u] = prolong_axis<n1, N>(x0 + u, wx[u]);
+    ly[u] = prolong_axis<n1, N>(y0 + u, wy[u]);
+  }
+#pragma unroll
+  for (int zi = 0; zi < M::H; zi++) {
+    T wz[2];
+    const int lz = prolong_axis<n1, N>(z0 + zi, wz);
+#pragma unroll
+    for (int yy = 0; yy < 2; yy++) {
+      const int xx = o.xx_of(ODD, yy, zi);
+      const T wzy[2][2] = {{wz[0] * wy[yy][0], wz[0] * wy[yy][1]}, {wz[1] * wy[yy][0], wz[1] * wy[yy][1]}};
+      o.phi[yy][xx][zi] = o.phi[yy][xx][zi] + prolong_cell<n1>(cs + cnat(n1, lx[xx], ly[yy], lz), wzy, wx[xx]);
+    }
+  }
+  o.template publish<ODD>(lds);
+}
+
 // Coarse level l and below: the correction for the right-hand side in rhs (the thread's cells), left in the level's
 // solution array.  Called by all threads, or by the first wave alone once a level fits it.
 template <int GS, int l, bool ONE_WAVE, typename PT, typename T = typename PT::real>
@@ -366,13 +401,15 @@ __device__ __forceinline__ void coarse_cycle(T* __restrict__ lds, const MgCoarse
   constexpr int n = M::n(l);
   const T dh = P.dh * T(M::N - 1) / T(n - 1), dh2 = dh * dh;
   T* sol = lds + M::off_sol(l);
-  if (k.active) sol[k.id] = T(0);
-  if (k.two) sol[k.id + 1] = T(0);
-  level_sync<ONE_WAVE>();
   if constexpr (l == M::NLV - 1) {
-    smooth_coarse<n, ONE_WAVE>(k, sol, rhs, dh2, M::L.nbottom);
+    smooth_coarse<n, ONE_WAVE, true>(k, sol, rhs, dh2, M::L.nbottom);
   } else {
-    smooth_coarse<n, ONE_WAVE>(k, sol, rhs, dh2, P.mg_npre);
+    if (P.mg_npre == 0) {
+      if (k.active) sol[k.id] = T(0);
+      if (k.two) sol[k.id + 1] = T(0);
+      level_sync<ONE_WAVE>();
+    }
+    smooth_coarse<n, ONE_WAVE, true>(k, sol, rhs, dh2, P.mg_npre);
     T* def = lds + M::off_def(l);
     const T m_dh2 = T(-1) / dh2;
 #pragma unroll
@@ -396,15 +433,18 @@ __device__ __forceinline__ void coarse_cycle(T* __restrict__ lds, const MgCoarse
     T wz[2], wy[2];
     const int lz = prolong_axis<nn, n>(k.z, wz), ly = prolong_axis<nn, n>(k.y, wy);
     const T wzy[2][2] = {{wz[0] * wy[0], wz[0] * wy[1]}, {wz[1] * wy[0], wz[1] * wy[1]}};
-#pragma unroll
-    for (int xx = 0; xx < k.K; xx++)
-      if (k.has(xx)) {
-        T wx[2];
-        const int lx = prolong_axis<nn, n>(k.x + xx, wx);
-        sol[k.id + xx] = sol[k.id + xx] + prolong_cell<nn>(cs + cnat(nn, lx, ly, lz), wzy, wx);
-      }
+    // the next sweep overwrites colour 1 from colour 0: only colour 0 is corrected, unless there is no sweep
+    auto correct = [&](int xx) {
+      T wx[2];
+      const int lx = prolong_axis<nn, n>(k.x + xx, wx);
+      sol[k.id + xx] = sol[k.id + xx] + prolong_cell<nn>(cs + cnat(nn, lx, ly, lz), wzy, wx);
+    };
+    const int odd = (k.x + k.y + k.z) & 1, x0 = k.K == 2 ? odd : 0;
+    const bool all = P.mg_npost == 0;
+    if (k.K == 2 ? k.has(x0) : k.active && (!odd || all)) correct(x0);
+    if (k.K == 2 && all && k.has(1 - x0)) correct(1 - x0);
     level_sync<ONE_WAVE>();
-    smooth_coarse<n, ONE_WAVE>(k, sol, rhs, dh2, P.mg_npost);
+    smooth_coarse<n, ONE_WAVE, false>(k, sol, rhs, dh2, P.mg_npost);
   }
 }
 
@@ -620,32 +660,10 @@ __device__ void mg_patch(T* __restrict__ lds, const T* __restrict__ rho, const T
       coarse_cycle<GS, 1, ONE1>(lds, k1, r1, P);
     }
     __syncthreads();
-    // prolongate, correct and publish again
-    {
-      const T* cs = lds + M::off_sol(1);
-      T wx[2][2], wy[2][2];
-      int lx[2], ly[2];
-      const int x0 = opaque(o.x0), y0 = opaque(o.y0), z0 = opaque(o.z0);
-#pragma unroll
-      for (int u = 0; u < 2; u++) {
-        lx[u] = prolong_axis<n1, N>(x0 + u, wx[u]);
-        ly[u] = prolong_axis<n1, N>(y0 + u, wy[u]);
-      }
-#pragma unroll
-      for (int zi = 0; zi < H; zi++) {
-        T wz[2];
-        const int lz = prolong_axis<n1, N>(z0 + zi, wz);
-#pragma unroll
-        for (int yy = 0; yy < 2; yy++) {
-          const T wzy[2][2] = {{wz[0] * wy[yy][0], wz[0] * wy[yy][1]}, {wz[1] * wy[yy][0], wz[1] * wy[yy][1]}};
-#pragma unroll
-          for (int xx = 0; xx < 2; xx++)
-            o.phi[yy][xx][zi] = o.phi[yy][xx][zi] + prolong_cell<n1>(cs + cnat(n1, lx[xx], ly[yy], lz), wzy, wx[xx]);
-        }
-      }
-      o.template publish<0>(lds);
-      o.template publish<1>(lds);
-    }
+    // Prolongate, correct and publish again.  The next sweep overwrites colour 1 from colour 0: only colour 0 is corrected,
+    // unless there is no sweep.
+    prolongate_level0<false>(o, lds);
+    if (P.mg_npost == 0) prolongate_level0<true>(o, lds);
     __syncthreads();
     for (int s = 0; s < P.mg_npost; s++) smooth_level0<GS>(o, lds, dh2);
     T sd = T(0), ss = T(0);
@@ -865,7 +883,7 @@ enum MgForm { kMgBlocks, kMgCells };
 template <int GS, MgForm F, typename T>
 struct MgLaunch {
   static constexpr int THREADS = F == kMgCells ? mg_cell_threads(GS) : MgGeo<GS>::THREADS;
-  static constexpr int WAVES = F == kMgCells ? (sizeof(T) == 8 ? 3 : 6) : mg_waves(GS, sizeof(T));
+  static constexpr int WAVES = F == kMgCells ? (sizeof(T) == 8 ? 2 : 6) : mg_waves(GS, sizeof(T));
   static constexpr size_t LDS = sizeof(T) * (MgGeo<GS>::FLOATS + (F == kMgCells ? MgGeo<GS>::N * MgGeo<GS>::N * MgGeo<GS>::N : 0));
 };
 
