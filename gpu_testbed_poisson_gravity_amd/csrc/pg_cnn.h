@@ -26,15 +26,15 @@ constexpr int kCnnInput = kCnnPadVox * kCnnChannels;         // bf16 values per 
 constexpr int kCnnOutputs = kCnnVox * kCnnOut;               // fp32 values per output
 
 // mode 0: first layer, 1: residual layer, 2: linear output layer (D)
-hipError_t cnn_conv_fwd(const uint16_t* X, const uint16_t* W, const float* b, uint16_t* Y, uint16_t* H, float* D,
-                        int n, int mode, hipStream_t s);
-hipError_t cnn_mse(const float* D, const float* T, float* dY, float* partial, int nvox, int nblocks, hipStream_t s);
-// Adds the residual term of the loss (weight w) to dY and to the nblocks loss partials cnn_mse wrote.
-hipError_t cnn_res_loss(const float* D, const float* T, float* dY, float* partial, int n, float w, int nblocks,
+hipError_t cnn_conv_fwd(const uint16_t* X, const uint16_t* W, const float* b, uint16_t* Y, float* D, int n, int mode,
                         hipStream_t s);
-hipError_t cnn_relu_bwd(const float* dY, const uint16_t* H, uint16_t* dH, size_t count, int nblocks, hipStream_t s);
-hipError_t cnn_conv_bwd_data(const uint16_t* dH, const uint16_t* WT, const float* dYres, float* dX, int n,
-                             hipStream_t s);
+// Forward, loss against T [n][8^3][8] (squared error, plus res_weight times the squared residual it leaves) and output
+// gradients: y[1..5] (borders untouched), dH [6][n][8^3][16] and cnn_train_blocks(n) loss partials (sums).
+constexpr int kCnnTrainBlocks = 256;   // one per CU
+int cnn_train_blocks(int n);
+hipError_t cnn_train_pass(const uint16_t* x0, const uint16_t* WL, const uint16_t* WT, const float* P, const float* T,
+                          uint16_t* const (&y)[kCnnLayers], uint16_t* dH, float* lossp, int n, float res_weight,
+                          hipStream_t s);
 // Weight and bias gradients of all layers from their inputs x [n][10^3][16] (x[0]: the packed input, x[l]: y_l) and
 // output gradients dH [6][n][8^3][16], into g (parameter order).  part: [6][cnn_grad_parts(n)][kCnnLayerParams] floats.
 int cnn_grad_parts(int n);
@@ -42,8 +42,8 @@ hipError_t cnn_weight_grad(const uint16_t* const (&x)[kCnnLayers], const uint16_
                            hipStream_t s);
 hipError_t cnn_adam(float* p, const float* g, float* m, float* v, int n, float lr, float b1, float b2, float eps,
                     float c1, float c2, hipStream_t s);
-// Wb: [6][16][kCnnKF] forward layout; WT: [6][16][432] per-tap transposed (input-gradient pass); WL: the forward
-// layout lane-major, [6][15 steps][64 lanes][8], what lane l reads at step c (the fused kernel's A operand)
+// Wb: [6][16][kCnnKF] forward layout; WL: the same lane-major, [6][15 steps][64 lanes][8], what lane l reads at step c (the
+// fused kernels' A operand); WT: lane-major, rows and channels exchanged and taps reversed (input gradient)
 hipError_t cnn_weight_copies(const float* P, uint16_t* Wb, uint16_t* WT, uint16_t* WL, hipStream_t s);
 hipError_t cnn_prep(const float* rho, const float* cpot, int n, int gs, float cst, int int_scheme, uint16_t* x,
                     float* scale, hipStream_t s);

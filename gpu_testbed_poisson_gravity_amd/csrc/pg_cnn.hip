@@ -28,7 +28,7 @@
 // Forward K order: 15 steps c = dz*5 + s; step c covers the in-plane positions 2s and 2s+1 (position
 // dy*3 + dx, 16 channels each) of tap plane dz; position 9 is a pad with zero weights whose A operand
 // repeats position 8.  Grouping the steps by dz lets the fused kernel read an input plane once and feed it
-// to the three output planes that use it.  The backward passes keep the tap-major order k = tap*16 + ci.
+// to the three output planes that use it.  The input gradient is the same convolution with the taps reversed.
 
 #include <hip/hip_runtime.h>
 
@@ -78,28 +78,12 @@ constexpr int S = kCnnPadded;   // 10: padded input edge
 constexpr int So = kCnnEdge;    // 8: output edge
 constexpr int CH = 16;          // channels
 constexpr int K = 27 * CH;      // 432
-constexpr int KC = (K + 31) / 32;  // 14 MFMA K-steps of the tap-major order (the last one half used)
 constexpr int KZ = 15;          // forward K steps: 3 dz x 5 position pairs
 constexpr int KF = KZ * 32;     // 480 = kCnnKF
 static_assert(KF == kCnnKF, "forward weight layout");
 constexpr int kTZ = 2;          // output z-planes per workgroup
 constexpr int kSlabs = So / kTZ;
 constexpr int kPlane = S * S * CH;  // bf16 values per padded plane
-
-// B operand (16 columns of a [16][432] weight matrix, row j = lane%16) for every K step.
-__device__ __forceinline__ void load_weights(const u16* __restrict__ W, bf16x8 (&wreg)[KC]) {
-  const int j = threadIdx.x & 15, kq = 8 * ((threadIdx.x & 63) >> 4);
-#pragma unroll
-  for (int c = 0; c < KC; c++) {
-    Pack8 p;
-    const int kb = c * 32 + kq;
-    if (kb < K)
-      p.u = *reinterpret_cast<const uint4*>(W + j * K + kb);
-    else
-      p.u = make_uint4(0, 0, 0, 0);
-    wreg[c] = p.v;
-  }
-}
 
 // Step c of this lane's A operand from the lane-major copy WL of one layer ([15][64][8]).
 __device__ __forceinline__ bf16x8 load_weight_step(const u16* __restrict__ WL, int c) {
@@ -119,18 +103,28 @@ __device__ __forceinline__ void load_weights_fwd(const u16* __restrict__ W, bf16
   }
 }
 
+// Activation buffers in LDS (the fused kernels): planes of [half][10 x 10 voxels][8 channels] BF16, the halves kHalfV
+// values apart.  A 16-byte read serves 16 lanes per cycle from 64 banks: lanes 0-3, 12-15 and 20-27 of each half wave, then
+// the others (measured; 16 consecutive lanes do not share a cycle).  So a tile of 16 voxels is rows r and r + 4 (640 bytes
+// apart) with lane j at x = tile_x(j), and the halves lie 1664 bytes apart: half a wave's lanes 0-3, 12-15 (half 0) and
+// 20-27 (half 1) then read 16 different bank quads.  With halves of 1600 bytes and x = j % 8 each read took 8 cycles or
+// more in place of 4.
+constexpr int kHalfV = S * S * 8 + 32;
+constexpr int kPlaneV = 2 * kHalfV;   // per plane
+__device__ __forceinline__ int tile_x(int j) { return (j & 7) ^ ((j & 8) >> 1); }
+__device__ __forceinline__ int tile_dy(int j) { return (j & 8) >> 1; }   // 0 or 4
+
 // In-plane position (dy*3 + dx) and channel half read by lane group g = lane/16 at position pair s.
 __device__ __forceinline__ int fwd_pos(int s, int g) { return min(2 * s + (g >> 1), 8); }
 
 // ---- forward convolution ------------------------------------------------------------------------------
 // MODE 0: y = relu(h) (layer 1);  MODE 1: y = x_centre + relu(h) (layers 2-5), both written into the
-// interior of a padded [n][10^3][16] BF16 buffer whose border stays zero, with h kept for the backward
-// pass when H != null;  MODE 2: D = h for the first 8 channels, FP32 [n][8^3][8] (output layer).
-// One workgroup: kTZ output planes of one sample.
+// interior of a padded [n][10^3][16] BF16 buffer whose border stays zero;  MODE 2: D = h for the first 8 channels,
+// FP32 [n][8^3][8] (output layer).  One workgroup: kTZ output planes of one sample.
 template <int MODE>
 __global__ void __launch_bounds__(kThreads) conv_fwd_kernel(const u16* __restrict__ X, const u16* __restrict__ W,
                                                             const float* __restrict__ bias, u16* __restrict__ Y,
-                                                            u16* __restrict__ H, float* __restrict__ D) {
+                                                            float* __restrict__ D) {
   __shared__ uint4 smem[(kTZ + 2) * kPlane / 8];
   const u16* xs = reinterpret_cast<const u16*>(smem);
   const int n = blockIdx.x / kSlabs, z0 = (blockIdx.x % kSlabs) * kTZ;
@@ -169,152 +163,306 @@ __global__ void __launch_bounds__(kThreads) conv_fwd_kernel(const u16* __restric
       }
       *reinterpret_cast<uint2*>(Y + ((((size_t)n * S + z0 + lz + 1) * S + oy + 1) * S + ox + 1) * CH + co0) =
           pack4_bf16(o0, o1, o2, o3);
-      if (H) *reinterpret_cast<uint2*>(H + o * CH + co0) = pack4_bf16(h0, h1, h2, h3);
     }
   }
 }
 
-// ---- loss and backward ---------------------------------------------------------------------------------
+// ---- training pass -----------------------------------------------------------------------------------------
 
-// MSE over the n*512*8 outputs: dY [n][512][16] = 2 (D - T) / count on the 8 live channels, 0 on the
-// others; per-block partial sums of (D - T)^2.
-__global__ void __launch_bounds__(kThreads) mse_kernel(const float* __restrict__ D, const float* __restrict__ T,
-                                                       float* __restrict__ dY, float* __restrict__ partial,
-                                                       int nvox) {
-  __shared__ float red[kThreads];
-  const float inv = 2.0f / ((float)nvox * kCnnOut);
-  float s = 0.0f;
-  for (int i = blockIdx.x * kThreads + threadIdx.x; i < nvox * CH; i += gridDim.x * kThreads) {
-    const int v = i / CH, c = i % CH;
-    float g = 0.0f;
-    if (c < kCnnOut) {
-      const float e = D[(size_t)v * kCnnOut + c] - T[(size_t)v * kCnnOut + c];
-      s += e * e;
-      g = e * inv;
-    }
-    dY[i] = g;
-  }
-  red[threadIdx.x] = s;
-  __syncthreads();
-  for (int o = kThreads / 2; o > 0; o >>= 1) {
-    if ((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) partial[blockIdx.x] = red[0];
+// Forward, loss and the gradients of every layer's output, one workgroup (16 waves) per sample: activations and output
+// gradients pass from layer to layer through two LDS buffers, each lane's own gradients and ReLU masks stay in its
+// registers, and memory only sees what weight_grad_kernel reads (y1..y5 and dH of every layer).
+//
+// The input gradient of a layer is the same padded convolution of dH with the weights transposed and its taps reversed,
+// so one routine serves both directions: weights are the A operand, and a lane has channels 4*(lane/16)..+3 of voxel
+// lane%16 of its wave's tiles.  A wave owns kTiles tiles one above the other in z (y rows r and r + 4) and walks the
+// kTiles + 2 input planes they need: 20 operand reads for 30 products, in the K order of conv_fwd_kernel.
+//
+// Buffers: ten planes with a zero border but for the packed input, whose border is the caller's.
+//
+// Loss: e = D - T, mean(e^2), and with res_weight the residual r = stencil(e) that the error leaves in the guess on the
+// 16^3 frame (fine cell 2o + p of output voxel o, sub-cell p): dY = 2 e / count + res_weight * 2 / count * stencil(r) (the
+// stencil is symmetric with the zero exterior).  One partial sum per workgroup.
+//
+// Bound by the chain of twelve short phases: with one sample per CU the LDS unit, the matrix cores and the VALU are each
+// busy for about a quarter of it; a third of the time is the launch and the 57 MB to and from memory.  MI355X, 256
+// samples: 35 us (512 threads 35.5 us; each wave loading its own weights 37 us with 512 threads and 43 us with 1024; with
+// the two-way conflicts of unpadded halves 44 us); 247 us as 19 launches (a layer each, the ReLU masks, the two terms of
+// the loss) that passed gradients and pre-activations through memory.
+constexpr int kTrainThreads = 1024;
+constexpr int kTiles = kCnnVox / 16 / (kTrainThreads / 64);   // per wave
+constexpr int kTBuf = S * kPlaneV;                   // u16 per buffer
+// FP32 frame of the loss with a zero halo.  Eight rows are 16 modulo 32 and the plane pitch is odd: the cells that half a
+// wave reads for its sub-cells (two y rows, two z planes, every other x) fall on 32 banks.
+constexpr int kFY = 18, kFZ = 18 * kFY + 1, kFrame = 18 * kFZ;
+struct TrainLds {
+  u16 a[kTBuf], b[kTBuf];              // packed input, activations, dH
+  u16 w[2][16 * KF];                   // weights of this layer and of the next, lane-major
+  float e[kFrame + 2], r[kFrame + 2];
+  float red[kTrainThreads / 64];
+};
+static_assert(sizeof(TrainLds) <= 160 * 1024 && sizeof(TrainLds) % 16 == 0, "one workgroup per CU");
+
+struct TrainOut {
+  u16* y[kCnnLayers];   // y[1..5]: layer outputs, padded [n][10^3][16]
+  u16* dh;              // [6][n][8^3][16]
+  float* loss;          // one partial per workgroup
+};
+
+// A value the compiler cannot see through: addresses derived from it are computed in each phase, not kept across them.
+__device__ __forceinline__ int opaque(int v) {
+  asm volatile("" : "+v"(v));
+  return v;
 }
 
-// 7-point stencil (six neighbours - 6 a) at cell f of a 16^3 frame held in LDS, zero outside the frame.
-__device__ __forceinline__ float stencil16(const float* a, int f) {
-  constexpr int F = 16;
-  const int x = f % F, y = (f / F) % F, z = f / (F * F);
-  const float zp = z + 1 < F ? a[f + F * F] : 0.0f, zm = z > 0 ? a[f - F * F] : 0.0f;
-  const float yp = y + 1 < F ? a[f + F] : 0.0f, ym = y > 0 ? a[f - F] : 0.0f;
-  const float xp = x + 1 < F ? a[f + 1] : 0.0f, xm = x > 0 ? a[f - 1] : 0.0f;
-  return (((((zp + zm) + yp) + ym) + xp) + xm) - 6.0f * a[f];
+// This lane's voxel of tile k is (z + k, y, x); its channels are co0..co0+3.
+struct TrainLane {
+  int z, y, x, co0;
+  __device__ __forceinline__ TrainLane() {
+    const int tid = opaque(threadIdx.x), wave = tid >> 6, lane = tid & 63;
+    z = kTiles * (wave >> 2);
+    y = (wave & 3) + tile_dy(lane);
+    x = tile_x(lane);
+    co0 = 4 * (lane >> 4);
+  }
+  // the four channels of tile k in a buffer (8 bytes)
+  __device__ __forceinline__ u16* at(u16* buf, int k) const {
+    return buf + (z + k + 1) * kPlaneV + (co0 >> 3) * kHalfV + ((y + 1) * S + x + 1) * 8 + (co0 & 7);
+  }
+  __device__ __forceinline__ int voxel(int k) const { return ((z + k) * So + y) * So + x; }
+  __device__ __forceinline__ int padded(int k) const { return ((z + k + 1) * S + y + 1) * S + x + 1; }
+};
+
+// Barrier for what the buffers hand over: the stores to memory, which only the next kernel reads, stay in flight.
+__device__ __forceinline__ void train_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// Residual term of the loss, run after mse_kernel on the same stream: per sample, e = D - T on the 16^3
-// frame (fine cell 2o + p of output voxel o, sub-cell p) and r = stencil(e), the residual the error leaves in
-// the guess.  Adds w * 2 / (n * 4096) * stencil(r) to dY (the stencil is symmetric with the zero exterior)
-// and w * sum(r^2) to this block's loss partial.  Block b handles samples b, b + gridDim.x, ...
-__global__ void __launch_bounds__(kThreads) res_loss_kernel(const float* __restrict__ D, const float* __restrict__ T,
-                                                            float* __restrict__ dY, float* __restrict__ partial,
-                                                            int n, float w) {
-  constexpr int F = 16, F3 = F * F * F;
-  static_assert(F3 == kCnnOutputs, "one frame cell per output value");
-  __shared__ float e[F3], r[F3];
-  __shared__ float red[kThreads];
-  const float k = w * (2.0f / ((float)n * kCnnOutputs));
-  float acc = 0.0f;
-  for (int smp = blockIdx.x; smp < n; smp += gridDim.x) {
-    const float* d = D + (size_t)smp * kCnnOutputs;
-    const float* t = T + (size_t)smp * kCnnOutputs;
-    for (int f = threadIdx.x; f < F3; f += kThreads) {
-      const int x = f % F, y = (f / F) % F, z = f / (F * F);
-      const int o = ((z >> 1) * So + (y >> 1)) * So + (x >> 1), p = ((z & 1) * 2 + (y & 1)) * 2 + (x & 1);
-      e[f] = d[o * kCnnOut + p] - t[o * kCnnOut + p];
-    }
-    __syncthreads();
-    for (int f = threadIdx.x; f < F3; f += kThreads) {
-      const float v = stencil16(e, f);
-      r[f] = v;
-      acc += v * v;
-    }
-    __syncthreads();
-    for (int f = threadIdx.x; f < F3; f += kThreads) {
-      const int x = f % F, y = (f / F) % F, z = f / (F * F);
-      const int o = ((z >> 1) * So + (y >> 1)) * So + (x >> 1), p = ((z & 1) * 2 + (y & 1)) * 2 + (x & 1);
-      dY[((size_t)smp * kCnnVox + o) * CH + p] += k * stencil16(r, f);
-    }
-    __syncthreads();   // e and r are rewritten for the next sample
-  }
-  red[threadIdx.x] = acc;
-  __syncthreads();
-  for (int o = kThreads / 2; o > 0; o >>= 1) {
-    if ((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) partial[blockIdx.x] += w * red[0];
-}
-
-// dH = dY * (H > 0) (or dY when H is null: the linear output layer), stored BF16 for the matrix cores.
-__global__ void __launch_bounds__(kThreads) relu_bwd_kernel(const float* __restrict__ dY, const u16* __restrict__ H,
-                                                            u16* __restrict__ dH, size_t count) {
-  for (size_t i = (size_t)blockIdx.x * kThreads + threadIdx.x; i < count; i += (size_t)gridDim.x * kThreads)
-    dH[i] = f2bf((H == nullptr || bf2f(H[i]) > 0.0f) ? dY[i] : 0.0f);
-}
-
-// Input gradient on the interior of the padded input: dX[p][ci] = sum_{tap,co} W[co][tap][ci] dH[p+1-tap][co]
-// (+ dYres[p][ci], the residual path), p in 8^3.  Implicit GEMM with WT[ci][tap*16+co].
-__global__ void __launch_bounds__(kThreads) conv_bwd_data_kernel(const u16* __restrict__ dH, const u16* __restrict__ WT,
-                                                                 const float* __restrict__ dYres,
-                                                                 float* __restrict__ dX) {
-  constexpr int pv = So * So * 2;  // uint4 per dH plane (16 channels = 2 x uint4)
-  __shared__ uint4 smem[(kTZ + 2) * pv];
-  const u16* hs = reinterpret_cast<const u16*>(smem);
-  const int n = blockIdx.x / kSlabs, z0 = (blockIdx.x % kSlabs) * kTZ;
-  // dH planes o_z in [z0-1, z0+kTZ], zero outside [0, So)
-  for (int i = threadIdx.x; i < (kTZ + 2) * pv; i += kThreads) {
-    const int pl = i / pv, r = i % pv;
-    const int qz = z0 - 1 + pl;
-    uint4 v = make_uint4(0, 0, 0, 0);
-    if (qz >= 0 && qz < So) v = reinterpret_cast<const uint4*>(dH + (((size_t)n * So + qz) * So * So) * CH)[r];
-    smem[i] = v;
-  }
-  bf16x8 wreg[KC];
-  load_weights(WT, wreg);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int ci = lane & 15, kq = 8 * (lane >> 4);
-  __syncthreads();
-  constexpr int M = kTZ * So * So;
-  for (int t = wave; t < M / 16; t += kThreads / 64) {
-    const int v = t * 16 + (lane & 15);
-    const int lz = v / (So * So), py = (v / So) % So, px = v % So;
-    floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+// A layer's weights: requested into registers one layer ahead, written to LDS when that layer ends, read by every wave.
+// (Each wave loading its 15 KB from L2 through the L1 was a quarter of the kernel.)
+constexpr int kWVec = 16 * KF / 8, kWFetch = (kWVec + kTrainThreads - 1) / kTrainThreads;
+__device__ __forceinline__ void train_fetch(const u16* __restrict__ W, int l, uint4 (&f)[kWFetch]) {
 #pragma unroll
-    for (int c = 0; c < KC; c++) {
-      const int kb = c * 32 + kq;
-      const int tap = kb / CH, co0 = kb % CH;
+  for (int j = 0; j < kWFetch; j++) {
+    const int i = threadIdx.x + j * kTrainThreads;
+    f[j] = i < kWVec ? reinterpret_cast<const uint4*>(W + (size_t)(l - 1) * 16 * KF)[i] : make_uint4(0, 0, 0, 0);
+  }
+}
+__device__ __forceinline__ void train_put(u16* w, const uint4 (&f)[kWFetch]) {
+#pragma unroll
+  for (int j = 0; j < kWFetch; j++) {
+    const int i = threadIdx.x + j * kTrainThreads;
+    if (i < kWVec) reinterpret_cast<uint4*>(w)[i] = f[j];
+  }
+}
+
+// Zero the border of the buffer that held the packed input.
+__device__ __forceinline__ void train_zero_border(u16* buf) {
+#pragma unroll 1
+  for (int i = opaque(threadIdx.x); i < kCnnPadVox * 2; i += kTrainThreads) {
+    const int vox = i >> 1, x = vox % S, y = vox / S % S, z = vox / (S * S);
+    if (x == 0 || x == S - 1 || y == 0 || y == S - 1 || z == 0 || z == S - 1)
+      *reinterpret_cast<uint4*>(buf + z * kPlaneV + (i & 1) * kHalfV + (y * S + x) * 8) = make_uint4(0, 0, 0, 0);
+  }
+}
+
+__device__ __forceinline__ float4 train_bias(const float* __restrict__ P, int l) {
+  return *reinterpret_cast<const float4*>(P + (size_t)(l - 1) * kCnnLayerParams + 16 * K + 4 * ((threadIdx.x & 63) >> 4));
+}
+
+__device__ __forceinline__ void train_conv(const u16* in, const u16* wl, floatx4 (&acc)[kTiles]) {
+  bf16x8 w[KZ];
+#pragma unroll
+  for (int c = 0; c < KZ; c++) w[c] = load_weight_step(wl, c);
+  const TrainLane t;
+  const int g = t.co0 >> 2;
+  const u16* base = in + t.z * kPlaneV + (g & 1) * kHalfV + (t.y * S + t.x) * 8;
+#pragma unroll
+  for (int k = 0; k < kTiles; k++) acc[k] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int p = 0; p < kTiles + 2; p++)
+#pragma unroll
+    for (int s = 0; s < 5; s++) {
+      const int pos = fwd_pos(s, g);
       Pack8 a;
-      a.u = make_uint4(0, 0, 0, 0);
-      if (tap < 27) {
-        const int dz = tap / 9, dy = (tap / 3) % 3, dx = tap % 3;
-        const int qy = py + 1 - dy, qx = px + 1 - dx;
-        // staged plane of o_z = z0 + lz + 1 - dz is lz + 2 - dz
-        if (qy >= 0 && qy < So && qx >= 0 && qx < So)
-          a.u = *reinterpret_cast<const uint4*>(hs + (((lz + 2 - dz) * So + qy) * So + qx) * CH + co0);
-      }
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.v, wreg[c], acc, 0, 0, 0);
-    }
+      a.u = *reinterpret_cast<const uint4*>(base + p * kPlaneV + ((pos / 3) * S + pos % 3) * 8);
 #pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const int vo = t * 16 + 4 * (lane >> 4) + r;
-      const int z = vo / (So * So), y = (vo / So) % So, x = vo % So;
-      const size_t o = ((((size_t)n * So + z0 + z) * So + y) * So + x) * CH + ci;
-      float g = acc[r];
-      if (dYres) g += dYres[o];
-      dX[o] = g;
+      for (int k = 0; k < kTiles; k++)
+        if (p >= k && p <= k + 2) acc[k] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[(p - k) * 5 + s], a.v, acc[k], 0, 0, 0);
     }
+}
+
+// Forward epilogue of layers 1..5: relu(h) (+ the layer's input) to the other buffer and to memory; returns the mask bits.
+__device__ __forceinline__ uint32_t train_relu(u16* in, u16* out, bool res, const floatx4 (&acc)[kTiles],
+                                               const float4& b, u16* __restrict__ Y) {
+  const TrainLane t;
+  uint32_t mask = 0;
+#pragma unroll
+  for (int k = 0; k < kTiles; k++) {
+    const float h0 = acc[k][0] + b.x, h1 = acc[k][1] + b.y, h2 = acc[k][2] + b.z, h3 = acc[k][3] + b.w;
+    const uint2 hb = pack4_bf16(h0, h1, h2, h3);   // the mask is that of the stored precision
+    mask |= ((uint32_t)(bf_lo(hb.x) > 0.0f) | (uint32_t)(bf_hi(hb.x) > 0.0f) << 1 | (uint32_t)(bf_lo(hb.y) > 0.0f) << 2 |
+             (uint32_t)(bf_hi(hb.y) > 0.0f) << 3)
+            << (4 * k);
+    float o0 = fmaxf(h0, 0.0f), o1 = fmaxf(h1, 0.0f), o2 = fmaxf(h2, 0.0f), o3 = fmaxf(h3, 0.0f);
+    uint2 rx = *reinterpret_cast<const uint2*>(t.at(in, k));
+    rx = res ? rx : make_uint2(0, 0);
+    o0 += bf_lo(rx.x);
+    o1 += bf_hi(rx.x);
+    o2 += bf_lo(rx.y);
+    o3 += bf_hi(rx.y);
+    const uint2 ob = pack4_bf16(o0, o1, o2, o3);
+    *reinterpret_cast<uint2*>(t.at(out, k)) = ob;
+    *reinterpret_cast<uint2*>(Y + t.padded(k) * CH + t.co0) = ob;
+  }
+  return opaque(mask);   // kept as bits, not as the 16 values they come from
+}
+
+// 7-point stencil (six neighbours - 6 a) at a cell of a frame.
+__device__ __forceinline__ float train_stencil(const float* a) {
+  return (((((a[kFZ] + a[-kFZ]) + a[kFY]) + a[-kFY]) + a[1]) + a[-1]) - 6.0f * a[0];
+}
+
+// Loss of the sample's output h6 = acc + b; dY of the lane's four channels (zero for the dead ones).
+__device__ __forceinline__ void train_loss(TrainLds& s, const floatx4 (&acc)[kTiles], const float4& b,
+                                           const float* __restrict__ T, float inv, float kr, bool res, float& se, float& sr,
+                                           float (&dy)[kTiles][4]) {
+  const TrainLane t;
+  const bool live = t.co0 < kCnnOut;   // sub-cells of z parity co0 / 4
+  const int f0 = (2 * t.z + (t.co0 >> 2 & 1) + 1) * kFZ + (2 * t.y + 1) * kFY + 2 * t.x + 1;
+#pragma unroll
+  for (int k = 0; k < kTiles; k++)
+#pragma unroll
+    for (int c = 0; c < 4; c++) dy[k][c] = 0.0f;
+  if (live) {
+#pragma unroll
+    for (int k = 0; k < kTiles; k++) {
+      const float* tv = T + t.voxel(k) * kCnnOut + t.co0;   // any alignment
+      const float d[4] = {(acc[k][0] + b.x) - tv[0], (acc[k][1] + b.y) - tv[1], (acc[k][2] + b.z) - tv[2], (acc[k][3] + b.w) - tv[3]};
+      float* ef = s.e + f0 + 2 * k * kFZ;
+#pragma unroll
+      for (int c = 0; c < 4; c++) {
+        se += d[c] * d[c];
+        dy[k][c] = d[c] * inv;
+        ef[(c >> 1) * kFY + (c & 1)] = d[c];
+      }
+    }
+  }
+  train_barrier();
+  if (!res) return;
+  constexpr int kPlanes = kTrainThreads / 256;   // per pass
+  const int q = opaque(threadIdx.x), fr = ((q >> 8) + 1) * kFZ + ((q >> 4 & 15) + 1) * kFY + (q & 15) + 1;
+#pragma unroll
+  for (int j = 0; j < 16 / kPlanes; j++) {
+    const int f = fr + kPlanes * j * kFZ;
+    const float v = train_stencil(s.e + f);
+    s.r[f] = v;
+    sr += v * v;
+  }
+  train_barrier();
+  if (live) {
+#pragma unroll
+    for (int k = 0; k < kTiles; k++)
+#pragma unroll
+      for (int c = 0; c < 4; c++) dy[k][c] += kr * train_stencil(s.r + f0 + 2 * k * kFZ + (c >> 1) * kFY + (c & 1));
+  }
+}
+
+// dH of a layer from dY and its mask bits, to a buffer and to memory.
+__device__ __forceinline__ void train_mask(const float (&dy)[kTiles][4], uint32_t mask, u16* out,
+                                           u16* __restrict__ dH) {
+  const TrainLane t;
+#pragma unroll
+  for (int k = 0; k < kTiles; k++) {
+    const uint32_t m = mask >> (4 * k);
+    const uint2 v = pack4_bf16(m & 1 ? dy[k][0] : 0.0f, m & 2 ? dy[k][1] : 0.0f, m & 4 ? dy[k][2] : 0.0f, m & 8 ? dy[k][3] : 0.0f);
+    *reinterpret_cast<uint2*>(t.at(out, k)) = v;
+    *reinterpret_cast<uint2*>(dH + t.voxel(k) * CH + t.co0) = v;
+  }
+}
+
+__global__ void __launch_bounds__(kTrainThreads, kTrainThreads / 256) train_pass_kernel(const u16* __restrict__ X0, const u16* __restrict__ WL,
+                                                                      const u16* __restrict__ WT, const float* __restrict__ P,
+                                                                      const float* __restrict__ T, int n, float res_weight,
+                                                                      TrainOut out) {
+  __shared__ __align__(16) TrainLds lds;
+  const float inv = 2.0f / ((float)(n * kCnnVox) * kCnnOut), kr = res_weight * (2.0f / ((float)n * kCnnOutputs));
+  float se = 0.0f, sr = 0.0f;
+  for (int i = threadIdx.x; i < (int)(sizeof(TrainLds) / 16); i += kTrainThreads)
+    reinterpret_cast<uint4*>(&lds)[i] = make_uint4(0, 0, 0, 0);
+  train_barrier();
+  for (int smp = blockIdx.x; smp < n; smp += gridDim.x) {
+    floatx4 acc[kTiles];
+    uint32_t mask1 = 0;   // ReLU masks: layer 1, and 16 bits each of layers 2..5 (5 lowest)
+    uint64_t masks = 0;
+    float dy[kTiles][4];
+    uint4 f[kWFetch];
+    train_fetch(WL, 1, f);
+    const uint4* src = reinterpret_cast<const uint4*>(X0 + (size_t)smp * kCnnInput);
+    for (int i = opaque(threadIdx.x); i < kCnnPadVox * 2; i += kTrainThreads) {
+      const int vox = i >> 1;
+      *reinterpret_cast<uint4*>(lds.a + vox / (S * S) * kPlaneV + (i & 1) * kHalfV + vox % (S * S) * 8) = src[i];
+    }
+    train_put(lds.w[1], f);
+    train_barrier();
+    // A layer reads one buffer and one weight buffer and writes the others; what is rewritten was last read before the
+    // barrier that ended the layer before.  Forward layer l has weights l & 1, backward layer l those of the other parity.
+    // The loops over layers stay rolled: a workgroup has one sample or few, and runs from a cold instruction cache.
+#pragma unroll 1
+    for (int l = 1; l < kCnnLayers; l++) {
+      u16 *in = l & 1 ? lds.a : lds.b, *o = l & 1 ? lds.b : lds.a;
+      const float4 b = train_bias(P, l);
+      train_fetch(WL, l + 1, f);
+      train_conv(in, lds.w[l & 1], acc);
+      if (l == 2) train_zero_border(lds.a);   // of the packed input
+      const uint32_t m = train_relu(in, o, l > 1, acc, b, out.y[l] + (size_t)smp * kCnnInput);
+      if (l == 1)
+        mask1 = m;
+      else
+        masks = masks << 16 | m;
+      train_put(lds.w[l + 1 & 1], f);
+      train_barrier();
+    }
+    const float4 b6 = train_bias(P, kCnnLayers);
+    train_fetch(WT, kCnnLayers, f);
+    train_conv(lds.b, lds.w[0], acc);
+    train_put(lds.w[1], f);
+    train_loss(lds, acc, b6, T + (size_t)smp * kCnnOutputs, inv, kr, res_weight > 0.0f, se, sr, dy);
+    const size_t layer = (size_t)n * kCnnVox * CH;
+    u16* dh = out.dh + (size_t)smp * kCnnVox * CH + (kCnnLayers - 1) * layer;
+    train_mask(dy, 0xffffu, lds.b, dh);
+    train_barrier();
+#pragma unroll
+    for (int k = 0; k < kTiles; k++)
+#pragma unroll
+      for (int c = 0; c < 4; c++) dy[k][c] = 0.0f;   // layer 6 has no residual path
+#pragma unroll 1
+    for (int l = kCnnLayers; l > 1; l--) {
+      u16 *in = l & 1 ? lds.a : lds.b, *o = l & 1 ? lds.b : lds.a;
+      if (l > 2) train_fetch(WT, l - 1, f);
+      train_conv(in, lds.w[l + 1 & 1], acc);
+#pragma unroll
+      for (int k = 0; k < kTiles; k++)
+#pragma unroll
+        for (int c = 0; c < 4; c++) dy[k][c] += acc[k][c];
+      dh -= layer;
+      train_mask(dy, l > 2 ? (uint32_t)masks : mask1, o, dh);
+      masks >>= 16;
+      if (l > 2) train_put(lds.w[l & 1], f);
+      train_barrier();
+    }
+  }
+  float s = se + res_weight * sr;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+  if ((threadIdx.x & 63) == 0) lds.red[threadIdx.x >> 6] = s;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    float sum = lds.red[0];
+    for (int i = 1; i < kTrainThreads / 64; i++) sum += lds.red[i];
+    out.loss[blockIdx.x] = sum;
   }
 }
 
@@ -484,25 +632,20 @@ __global__ void adam_kernel(float* __restrict__ p, const float* __restrict__ g, 
 // BF16 copies of the six weight matrices: the forward layout Wb[l][co][c*32 + kk] (step c = dz*5 + s,
 // position 2s + kk/16, channel kk%16; zero at the pad position 9), the same values lane-major
 // WL[l][c][lane][8] (lane = co + 16*(kk/8) reads kk%8 = 0..7 of its row: one contiguous 1 KB load per step),
-// and per-tap transposed WT[l][ci][tap*16+co] = W[l][co][tap*16+ci] for the input-gradient pass.
+// and lane-major WT: rows and channels exchanged, taps reversed (W[l][kk%16][26 - tap][row]), for the input gradient.
 __global__ void weight_copies_kernel(const float* __restrict__ P, u16* __restrict__ Wb, u16* __restrict__ WT,
                                      u16* __restrict__ WL) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < kCnnLayers * 16 * KF) {
-    const int l = i / (16 * KF), r = i % (16 * KF);
-    const int co = r / KF, k = r % KF, c = k / 32, kk = k % 32;
-    const int dz = c / 5, pos = 2 * (c % 5) + (kk >> 4);
-    const float* W = P + (size_t)l * kCnnLayerParams;
-    const u16 v = pos < 9 ? f2bf(W[co * K + (dz * 9 + pos) * CH + (kk & 15)]) : (u16)0;
-    Wb[i] = v;
-    WL[(((size_t)l * KZ + c) * 64 + co + 16 * (kk >> 3)) * 8 + (kk & 7)] = v;
-  }
-  if (i < kCnnLayers * 16 * K) {
-    const int l = i / (16 * K), r = i % (16 * K);
-    const float* W = P + (size_t)l * kCnnLayerParams;
-    const int ci = r / K, k = r % K, tap = k / CH, co = k % CH;
-    WT[i] = f2bf(W[co * K + tap * CH + ci]);
-  }
+  if (i >= kCnnLayers * 16 * KF) return;
+  const int l = i / (16 * KF), r = i % (16 * KF);
+  const int row = r / KF, k = r % KF, c = k / 32, kk = k % 32;
+  const int dz = c / 5, pos = 2 * (c % 5) + (kk >> 4), tap = dz * 9 + pos, ch = kk & 15;
+  const float* W = P + (size_t)l * kCnnLayerParams;
+  const u16 v = pos < 9 ? f2bf(W[row * K + tap * CH + ch]) : (u16)0;
+  const size_t lm = (((size_t)l * KZ + c) * 64 + row + 16 * (kk >> 3)) * 8 + (kk & 7);
+  Wb[i] = v;
+  WL[lm] = v;
+  WT[lm] = pos < 9 ? f2bf(W[ch * K + (26 - tap) * CH + row]) : (u16)0;
 }
 
 // ---- input preparation and guess assembly -------------------------------------------------------------
@@ -638,9 +781,7 @@ __global__ void __launch_bounds__(kThreads) guess_kernel(const float* __restrict
 // that of prep + forward + guess with the layer-by-layer kernels.
 //
 // * An activation buffer holds only the 8 planes of the output grid, each [half][10 x 10 voxels][8 channels]
-//   BF16 with a zero ring (y or x = 0 or 9), 25.6 KB.  The 16-byte A-operand reads of 8 lanes (8 consecutive
-//   voxels along x) are one 128-byte span; a tile pairs rows r and r + 4, 640 bytes apart (128 modulo the
-//   256-byte bank width), so the 16 lanes of a read phase cover all 64 banks once.
+//   BF16 with a zero ring (y or x = 0 or 9), 26.6 KB.
 // * The packed input (the solve interior only; its border voxels are zero like the activations' padding)
 //   has the same layout, so the first layer is a layer like the others.
 // * Wave w owns output rows w and w + 4 of every plane and sweeps the 8 input planes once; every A operand
@@ -649,9 +790,7 @@ __global__ void __launch_bounds__(kThreads) guess_kernel(const float* __restrict
 // * Two buffers only: the coarse staging, the packed input and the activations share them with the FP32
 //   interpolated cube.  The interpolated values the guess adds to are written to the guess array while the
 //   input is packed; the output layer's epilogue reads them back (same lane, same address: L2), adds s * D and
-//   stores the guess.  LDS per workgroup 51.2 KB: three workgroups per CU.
-constexpr int kHalfV = S * S * 8;      // bf16 per half-plane (10 x 10 voxels x 8 channels)
-constexpr int kPlaneV = 2 * kHalfV;    // bf16 per plane
+//   stores the guess.  LDS per workgroup 53.3 KB: three workgroups per CU.
 constexpr int kActVec = So * kPlaneV / 8;   // uint4 per buffer (8 planes)
 constexpr int kCoarseMax = 12 * 12 * 12;    // C^3 at ghost size 5
 constexpr int kCubeMax = 18 * 18 * 18;      // N^3 at ghost size 5
@@ -727,7 +866,7 @@ __device__ __forceinline__ void conv_store(const u16* in, u16* out, const floatx
                                            const GuessOut& go) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int co0 = 4 * (lane >> 4);
-  const int row = wave + 4 * ((lane & 15) >> 3), xv = lane & 7;
+  const int row = wave + tile_dy(lane), xv = tile_x(lane);
   const float h0 = acc[0] + b.x, h1 = acc[1] + b.y, h2 = acc[2] + b.z, h3 = acc[3] + b.w;
   if (MODE == 2) {
     if (co0 < kCnnOut) {
@@ -765,8 +904,8 @@ __device__ __forceinline__ void conv_store(const u16* in, u16* out, const floatx
 template <int GS, bool CUBE, int MODE>
 __device__ __forceinline__ void conv_layer(const u16* in, u16* out, bf16x8 (&w)[KZ], const float4& b,
                                            const int (&off)[5], const GuessOut& go, const u16* __restrict__ Wn) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i = lane & 15;
-  const u16* col = in + ((wave + 4 * (i >> 3)) * S + (i & 7)) * 8;   // padded row = output row + dy
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const u16* col = in + ((wave + tile_dy(lane)) * S + tile_x(lane)) * 8;   // padded row = output row + dy
   const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
   floatx4 a0 = zero, a1 = zero;   // output planes z - 1 and z
   Pack8 nx[5];
@@ -1008,39 +1147,32 @@ __global__ void __launch_bounds__(kFT, kFusedBlocksPerCU) fused_guess_mixed_kern
 
 using namespace cnn;
 
-hipError_t cnn_conv_fwd(const uint16_t* X, const uint16_t* W, const float* b, uint16_t* Y, uint16_t* H, float* D,
-                        int n, int mode, hipStream_t s) {
+hipError_t cnn_conv_fwd(const uint16_t* X, const uint16_t* W, const float* b, uint16_t* Y, float* D, int n, int mode,
+                        hipStream_t s) {
   const dim3 grid(n * kSlabs), block(kThreads);
   if (mode == 0)
-    hipLaunchKernelGGL(conv_fwd_kernel<0>, grid, block, 0, s, X, W, b, Y, H, D);
+    hipLaunchKernelGGL(conv_fwd_kernel<0>, grid, block, 0, s, X, W, b, Y, D);
   else if (mode == 1)
-    hipLaunchKernelGGL(conv_fwd_kernel<1>, grid, block, 0, s, X, W, b, Y, H, D);
+    hipLaunchKernelGGL(conv_fwd_kernel<1>, grid, block, 0, s, X, W, b, Y, D);
   else if (mode == 2)
-    hipLaunchKernelGGL(conv_fwd_kernel<2>, grid, block, 0, s, X, W, b, Y, H, D);
+    hipLaunchKernelGGL(conv_fwd_kernel<2>, grid, block, 0, s, X, W, b, Y, D);
   else
     return hipErrorInvalidValue;
   return hipGetLastError();
 }
 
-hipError_t cnn_mse(const float* D, const float* T, float* dY, float* partial, int nvox, int nblocks, hipStream_t s) {
-  hipLaunchKernelGGL(mse_kernel, dim3(nblocks), dim3(kThreads), 0, s, D, T, dY, partial, nvox);
-  return hipGetLastError();
-}
+int cnn_train_blocks(int n) { return n < kCnnTrainBlocks ? n : kCnnTrainBlocks; }
 
-hipError_t cnn_res_loss(const float* D, const float* T, float* dY, float* partial, int n, float w, int nblocks,
-                        hipStream_t s) {
-  hipLaunchKernelGGL(res_loss_kernel, dim3(nblocks), dim3(kThreads), 0, s, D, T, dY, partial, n, w);
-  return hipGetLastError();
-}
-
-hipError_t cnn_relu_bwd(const float* dY, const uint16_t* H, uint16_t* dH, size_t count, int nblocks, hipStream_t s) {
-  hipLaunchKernelGGL(relu_bwd_kernel, dim3(nblocks), dim3(kThreads), 0, s, dY, H, dH, count);
-  return hipGetLastError();
-}
-
-hipError_t cnn_conv_bwd_data(const uint16_t* dH, const uint16_t* WT, const float* dYres, float* dX, int n,
-                             hipStream_t s) {
-  hipLaunchKernelGGL(conv_bwd_data_kernel, dim3(n * kSlabs), dim3(kThreads), 0, s, dH, WT, dYres, dX);
+hipError_t cnn_train_pass(const uint16_t* x0, const uint16_t* WL, const uint16_t* WT, const float* P, const float* T,
+                          uint16_t* const (&y)[kCnnLayers], uint16_t* dH, float* lossp, int n, float res_weight,
+                          hipStream_t s) {
+  TrainOut out;
+  for (int l = 1; l < kCnnLayers; l++) out.y[l] = y[l];
+  out.y[0] = nullptr;
+  out.dh = dH;
+  out.loss = lossp;
+  hipLaunchKernelGGL(train_pass_kernel, dim3(cnn_train_blocks(n)), dim3(kTrainThreads), 0, s, x0, WL, WT, P, T, n,
+                     res_weight, out);
   return hipGetLastError();
 }
 
@@ -1064,7 +1196,7 @@ hipError_t cnn_adam(float* p, const float* g, float* m, float* v, int n, float l
 }
 
 hipError_t cnn_weight_copies(const float* P, uint16_t* Wb, uint16_t* WT, uint16_t* WL, hipStream_t s) {
-  const int n = kCnnLayers * 16 * KF;   // covers every copy (KF > K)
+  const int n = kCnnLayers * 16 * KF;
   hipLaunchKernelGGL(weight_copies_kernel, dim3((n + 255) / 256), dim3(256), 0, s, P, Wb, WT, WL);
   return hipGetLastError();
 }

@@ -26,8 +26,6 @@ namespace {
 
 constexpr int kW = kCnnChannels * kCnnK;   // weights per layer
 constexpr int kWF = kCnnChannels * kCnnKF; // forward-layout BF16 weights per layer
-constexpr int kMseBlocks = 64;
-constexpr int kMaxReduceBlocks = 4096;
 constexpr int kMaxChunks = 16;               // pgamd_cnn_solve_device
 
 int ow(int l) { return (l - 1) * kCnnLayerParams; }   // layer l = 1..6
@@ -41,15 +39,14 @@ struct pgamd_cnn {
   float res_weight = 0.0f;  // weight of the residual term of the loss (pgamd_cnn_set_loss)
   float *p = nullptr, *g = nullptr, *m = nullptr, *v = nullptr;
   uint16_t* wb = nullptr;   // BF16 W1..W6 in the forward layout [16][480]
-  uint16_t* wt = nullptr;   // BF16 W1..W6 transposed per tap (input-gradient pass)
-  uint16_t* wl = nullptr;   // BF16 W1..W6 forward layout, lane-major (the fused warm-start kernel)
+  uint16_t* wt = nullptr;   // BF16 W1..W6 transposed, taps reversed, lane-major (input gradients)
+  uint16_t* wl = nullptr;   // BF16 W1..W6 forward layout, lane-major (the fused kernels)
   // workspace
   int cap = 0;              // samples
   bool train_ws = false;
   uint16_t* y[6] = {};      // y1..y5, padded [n][10^3][16] with zero borders (y[0] unused: the input)
-  uint16_t* h[6] = {};      // pre-activations h1..h5 [n][8^3][16] (training only)
   uint16_t* dh = nullptr;   // output gradients of the six layers, [6][n][8^3][16]
-  float *d = nullptr, *dy6 = nullptr, *dyA = nullptr, *dyB = nullptr, *part = nullptr, *lossp = nullptr;
+  float *d = nullptr, *part = nullptr, *lossp = nullptr;
   // pipelined warm-start solve: fork event and one event per chunk
   hipEvent_t ev[kMaxChunks + 1] = {};
 };
@@ -59,23 +56,17 @@ namespace {
 void free_ws(pgamd_cnn* n) {
   for (int l = 1; l <= 5; l++) {
     hipFree(n->y[l]);
-    hipFree(n->h[l]);
-    n->y[l] = n->h[l] = nullptr;
+    n->y[l] = nullptr;
   }
   hipFree(n->dh);
   hipFree(n->d);
-  hipFree(n->dy6);
-  hipFree(n->dyA);
-  hipFree(n->dyB);
   hipFree(n->part);
   hipFree(n->lossp);
   n->dh = nullptr;
-  n->d = n->dy6 = n->dyA = n->dyB = n->part = n->lossp = nullptr;
+  n->d = n->part = n->lossp = nullptr;
   n->cap = 0;
   n->train_ws = false;
 }
-
-int reduce_blocks(size_t elems) { return (int)std::min<size_t>((elems + 255) / 256, kMaxReduceBlocks); }
 
 int ensure_ws(pgamd_cnn* n, int count, bool train) {
   if (count <= n->cap && (!train || n->train_ws)) return PGAMD_OK;
@@ -87,16 +78,12 @@ int ensure_ws(pgamd_cnn* n, int count, bool train) {
     const size_t e = c * kCnnInput;
     ok &= hipMalloc(&n->y[l], e * 2) == hipSuccess;
     if (ok) ok &= hipMemset(n->y[l], 0, e * 2) == hipSuccess;   // borders stay zero for good
-    if (train) ok &= hipMalloc(&n->h[l], act * 2) == hipSuccess;
   }
   ok &= hipMalloc(&n->d, c * kCnnOutputs * 4) == hipSuccess;
   if (train) {
     ok &= hipMalloc(&n->dh, kCnnLayers * act * 2) == hipSuccess;
-    ok &= hipMalloc(&n->dy6, act * 4) == hipSuccess;
-    ok &= hipMalloc(&n->dyA, act * 4) == hipSuccess;
-    ok &= hipMalloc(&n->dyB, act * 4) == hipSuccess;
     ok &= hipMalloc(&n->part, (size_t)kCnnLayers * cnn_grad_parts(count) * kCnnLayerParams * 4) == hipSuccess;
-    ok &= hipMalloc(&n->lossp, kMseBlocks * 4) == hipSuccess;
+    ok &= hipMalloc(&n->lossp, cnn_train_blocks(count) * 4) == hipSuccess;
   }
   if (!ok) {
     free_ws(n);
@@ -118,51 +105,33 @@ int refresh_copies(pgamd_cnn* n, hipStream_t s) {
   return PGAMD_OK;
 }
 
-int forward(pgamd_cnn* n, const uint16_t* x0, int count, bool keep_h, hipStream_t s) {
+int forward(pgamd_cnn* n, const uint16_t* x0, int count, hipStream_t s) {
   const uint16_t* in = x0;
   for (int l = 1; l <= 5; l++) {
-    CK(cnn_conv_fwd(in, n->wb + (size_t)(l - 1) * kWF, n->p + ob(l), n->y[l], keep_h ? n->h[l] : nullptr, nullptr,
-                    count, l == 1 ? 0 : 1, s));
+    CK(cnn_conv_fwd(in, n->wb + (size_t)(l - 1) * kWF, n->p + ob(l), n->y[l], nullptr, count, l == 1 ? 0 : 1, s));
     in = n->y[l];
   }
-  CK(cnn_conv_fwd(in, n->wb + (size_t)5 * kWF, n->p + ob(6), nullptr, nullptr, n->d, count, 2, s));
+  CK(cnn_conv_fwd(in, n->wb + (size_t)5 * kWF, n->p + ob(6), nullptr, n->d, count, 2, s));
   return PGAMD_OK;
 }
 
 // Forward + backward; gradients (mean squared error, plus the residual term when res_weight > 0) go to n->g,
 // loss partials to lossp.
 int forward_backward(pgamd_cnn* n, const uint16_t* x0, const float* target, int count, hipStream_t s) {
-  int rc = forward(n, x0, count, true, s);
-  if (rc != PGAMD_OK) return rc;
-  const size_t act = (size_t)count * kCnnVox * kCnnChannels;
-  const int nb = reduce_blocks(act);
-  CK(cnn_mse(n->d, target, n->dy6, n->lossp, count * kCnnVox, kMseBlocks, s));
-  if (n->res_weight > 0.0f) CK(cnn_res_loss(n->d, target, n->dy6, n->lossp, count, n->res_weight, kMseBlocks, s));
-  const float* dy = n->dy6;
-  float* bufs[2] = {n->dyA, n->dyB};
-  int which = 0;
-  for (int l = 6; l >= 1; l--) {
-    uint16_t* dh = n->dh + (size_t)(l - 1) * act;
-    CK(cnn_relu_bwd(dy, l == 6 ? nullptr : n->h[l], dh, act, nb, s));
-    if (l > 1) {
-      float* dx = bufs[which];
-      which ^= 1;
-      CK(cnn_conv_bwd_data(dh, n->wt + (size_t)(l - 1) * kW, l == 6 ? nullptr : dy, dx, count, s));
-      dy = dx;
-    }
-  }
+  CK(cnn_train_pass(x0, n->wl, n->wt, n->p, target, n->y, n->dh, n->lossp, count, n->res_weight, s));
   const uint16_t* x[kCnnLayers] = {x0, n->y[1], n->y[2], n->y[3], n->y[4], n->y[5]};
   CK(cnn_weight_grad(x, n->dh, count, n->part, n->g, s));
   return PGAMD_OK;
 }
 
 float read_loss(pgamd_cnn* n, int count, hipStream_t s) {
-  float h[kMseBlocks];
-  if (hipMemcpyAsync(h, n->lossp, sizeof(h), hipMemcpyDeviceToHost, s) != hipSuccess ||
+  float h[kCnnTrainBlocks];
+  const int parts = cnn_train_blocks(count);
+  if (hipMemcpyAsync(h, n->lossp, parts * sizeof(float), hipMemcpyDeviceToHost, s) != hipSuccess ||
       hipStreamSynchronize(s) != hipSuccess)
     return NAN;
   double t = 0.0;
-  for (float x : h) t += x;
+  for (int i = 0; i < parts; i++) t += h[i];
   return (float)(t / ((double)count * kCnnOutputs));
 }
 
@@ -194,7 +163,7 @@ int pgamd_cnn_create(pgamd_context* ctx, uint64_t seed, pgamd_cnn** out) {
   if (hipSetDevice(n->device) != hipSuccess || hipMalloc(&n->p, kCnnParams * 4) != hipSuccess ||
       hipMalloc(&n->g, kCnnParams * 4) != hipSuccess || hipMalloc(&n->m, kCnnParams * 4) != hipSuccess ||
       hipMalloc(&n->v, kCnnParams * 4) != hipSuccess || hipMalloc(&n->wb, kCnnLayers * kWF * 2) != hipSuccess ||
-      hipMalloc(&n->wt, kCnnLayers * kW * 2) != hipSuccess || hipMalloc(&n->wl, kCnnLayers * kWF * 2) != hipSuccess) {
+      hipMalloc(&n->wt, kCnnLayers * kWF * 2) != hipSuccess || hipMalloc(&n->wl, kCnnLayers * kWF * 2) != hipSuccess) {
     pgamd_cnn_destroy(n);
     return set_error(PGAMD_ERR_NOMEM, "CNN parameter allocation failed");
   }
@@ -264,7 +233,7 @@ int pgamd_cnn_forward(pgamd_cnn* n, const uint16_t* d_x0, int count, float* d_ou
   hipStream_t s = (hipStream_t)stream;
   int rc = ensure_ws(n, count, n->train_ws && count <= n->cap);
   if (rc != PGAMD_OK) return rc;
-  rc = forward(n, d_x0, count, false, s);
+  rc = forward(n, d_x0, count, s);
   if (rc != PGAMD_OK) return rc;
   CK(hipMemcpyAsync(d_out, n->d, (size_t)count * kCnnOutputs * 4, hipMemcpyDeviceToDevice, s));
   return PGAMD_OK;

@@ -79,7 +79,7 @@ extern "C" int pgamd_cnn_forward_noalloc(pgamd_cnn* net, const uint16_t* d_x0, i
   const uint16_t* in = d_x0;
   for (int l = 1; l <= 6; l++) {
     const hipError_t e = cnn_conv_fwd(in, cnn_forward_weights(net, l), cnn_bias(net, l), l < 6 ? y[l] : nullptr,
-                                      nullptr, l < 6 ? nullptr : d_out, count, l == 1 ? 0 : (l < 6 ? 1 : 2), s);
+                                      l < 6 ? nullptr : d_out, count, l == 1 ? 0 : (l < 6 ? 1 : 2), s);
     if (e != hipSuccess) return set_error(PGAMD_ERR_DEVICE, hipGetErrorString(e));
     if (l < 6) in = y[l];
   }
