@@ -117,6 +117,8 @@ SolveParams make_params(const pgamd_options& o, const pgamd_solver_args& a) {
 
 }  // namespace pgamd
 
+constexpr int kSlicePatches = 512, kMaxSlices = 8;
+
 struct pgamd_context {
   int device = 0;
   hipDeviceProp_t prop{};
@@ -138,6 +140,8 @@ struct pgamd_context {
   hipStream_t aux = nullptr;                // forked launches (mixed batches)
   hipStream_t capture = nullptr;            // graph capture
   hipEvent_t ev[2] = {nullptr, nullptr};    // fork / join
+  hipStream_t copy[2] = {};                 // copies in / out of a sliced batch
+  hipEvent_t slice_ev[1 + 2 * kMaxSlices] = {};   // fork and join, then copied in and solved per slice
 };
 
 namespace {
@@ -164,6 +168,14 @@ int ensure_streams(pgamd_context* c, int n) {
     HIP_TRY(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
     c->streams.push_back(s);
   }
+  return PGAMD_OK;
+}
+
+int ensure_slices(pgamd_context* c) {
+  for (auto& s : c->copy)
+    if (!s) HIP_TRY(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
+  for (auto& e : c->slice_ev)
+    if (!e) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   return PGAMD_OK;
 }
 
@@ -232,6 +244,10 @@ int pgamd_destroy(pgamd_context* c) {
   if (c->capture) hipStreamDestroy(c->capture);
   for (auto e : c->ev)
     if (e) hipEventDestroy(e);
+  for (auto s : c->copy)
+    if (s) hipStreamDestroy(s);
+  for (auto e : c->slice_ev)
+    if (e) hipEventDestroy(e);
   delete c;
   return PGAMD_OK;
 }
@@ -274,6 +290,13 @@ int pgamd_mem_allocate_poisson_gravity(pgamd_context* c, int npatch_group, float
     return fail(PGAMD_ERR_NOMEM, "device/pinned allocation for %zu patches failed", np);
   }
   c->cap = (int)np;
+  if (c->cap >= 2 * kSlicePatches) {
+    const int rc = ensure_slices(c);
+    if (rc != PGAMD_OK) {
+      free_device(c);
+      return rc;
+    }
+  }
   // pinned host buffers handed to the caller (CUAPI_MemAllocate_PoissonGravity.cu:66-69)
   float** outs[4] = {h_rho, h_pot_in, h_pot_out, h_flu};
   const size_t sizes[4] = {np * c->rho_n * 4, np * c->cpot_n * 4, np * c->out_n * 4, np * flu_n * 4};
@@ -344,10 +367,7 @@ int pgamd_asyn_poisson_gravity_solver(pgamd_context* c, const float* h_rho, floa
   }
   count[gpu_nstream - 1] = npatch - first[gpu_nstream - 1];
 
-  for (int s = 0; s < gpu_nstream; s++) {  // a. host -> device
-    if (count[s] == 0) continue;
-    hipStream_t st = c->streams[s];
-    const size_t f = first[s], n = count[s];
+  auto copy_in = [&](size_t f, size_t n, hipStream_t st) -> int {
     if (poisson) {
       HIP_TRY(hipMemcpyAsync(c->d_rho + f * c->rho_n, h_rho + f * c->rho_n, n * c->rho_n * 4, hipMemcpyHostToDevice, st));
       HIP_TRY(hipMemcpyAsync(c->d_pot_in + f * c->cpot_n, h_pot_in + f * c->cpot_n, n * c->cpot_n * 4,
@@ -359,27 +379,86 @@ int pgamd_asyn_poisson_gravity_solver(pgamd_context* c, const float* h_rho, floa
                                hipMemcpyHostToDevice, st));
       HIP_TRY(hipMemcpyAsync(c->d_flu + f * flu_n, h_flu + f * flu_n, n * flu_n * 4, hipMemcpyHostToDevice, st));
     }
+    return PGAMD_OK;
+  };
+  auto solve = [&](size_t f, size_t n, hipStream_t st) -> int {
+    return pgamd::enqueue_solve(c, c->d_rho + f * c->rho_n, c->d_pot_in + f * c->cpot_n, nullptr,
+                                c->d_pot_out + f * c->out_n, graacc ? c->d_flu + f * flu_n : nullptr, (int)n, a, p,
+                                c->d_iters + f, c->d_status + f, st);
+  };
+  auto copy_out = [&](size_t f, size_t n, hipStream_t st) -> int {
+    if (poisson)
+      HIP_TRY(hipMemcpyAsync(h_pot_out + f * c->out_n, c->d_pot_out + f * c->out_n, n * c->out_n * 4,
+                             hipMemcpyDeviceToHost, st));
+    if (graacc)
+      HIP_TRY(hipMemcpyAsync(h_flu + f * flu_n, c->d_flu + f * flu_n, n * flu_n * 4, hipMemcpyDeviceToHost, st));
+    return PGAMD_OK;
+  };
+  auto copy_stats = [&](size_t f, size_t n, hipStream_t st) -> int {
+    if (!poisson) return PGAMD_OK;
+    HIP_TRY(hipMemcpyAsync(c->h_iters + f, c->d_iters + f, n * 4, hipMemcpyDeviceToHost, st));
+    HIP_TRY(hipMemcpyAsync(c->h_status + f, c->d_status + f, n * 4, hipMemcpyDeviceToHost, st));
+    return PGAMD_OK;
+  };
+
+  // One stream and a large batch: slices of n/2, n/4, ... patches, so that the copies of one hide behind the others.  The
+  // copies in follow each other without a gap and bound the call (33 KB a patch at ghost size 5, 57 GB/s); each slice is
+  // solved and copied out while the next half is on its way in, and the last one leaves a short tail.  Few slices, because
+  // every copy costs 10 to 15 us besides its bytes.  Copies run on two streams of the context's own, forked from the call's
+  // stream and joined to it at the end, so that later work on that stream (the next call's copies into the same device
+  // buffers) and pgamd_synchronize see the order of the plain sequence.  No slice is smaller than kSlicePatches, and slices
+  // begin at a multiple of every patches-per-wavefront layout.
+  // Ghost size 5, sequence -> slices: 512 patches 585 us either way, 1024 1.08 -> 1.02 ms, 2048 1.97 -> 1.69, 4096 3.83 ->
+  // 3.01 (8 equal slices 3.17), 16384 14.9 -> 10.8; the copies in alone take 2.4 ms at 4096.  Two streams of copies in share a
+  // hardware queue with the solves (3.74 ms), and copying out by a kernel of 16 workgroups gains 1%.
+  // Host arrays that share memory (other than the fluid with itself) keep the sequence: an early slice's results would
+  // overwrite what a later one reads.
+  auto apart = [&](const float* x, size_t xn, const float* y, size_t yn) {
+    const uintptr_t a0 = (uintptr_t)x, b0 = (uintptr_t)y;
+    return !x || !y || a0 + 4 * npatch * xn <= b0 || b0 + 4 * npatch * yn <= a0;
+  };
+  if (gpu_nstream == 1 && npatch >= 2 * kSlicePatches && apart(h_pot_out, c->out_n, h_rho, c->rho_n) &&
+      apart(h_pot_out, c->out_n, h_pot_in, c->cpot_n) && apart(h_pot_out, c->out_n, h_flu, flu_n) &&
+      apart(h_flu, flu_n, h_rho, c->rho_n) && apart(h_flu, flu_n, h_pot_in, c->cpot_n)) {
+    size_t at[kMaxSlices + 1] = {};
+    int ns = 0;
+    while (ns + 1 < kMaxSlices && npatch - at[ns] >= 2 * kSlicePatches) {
+      at[ns + 1] = at[ns] + (npatch - at[ns]) / 2 / 64 * 64;
+      ns++;
+    }
+    at[++ns] = npatch;
+    hipStream_t st = c->streams[0], in = c->copy[0], out = c->copy[1];
+    HIP_TRY(hipEventRecord(c->slice_ev[0], st));
+    HIP_TRY(hipStreamWaitEvent(in, c->slice_ev[0], 0));
+    for (int i = 0; i < ns; i++) {
+      const size_t f = at[i], n = at[i + 1] - f;
+      if ((rc = copy_in(f, n, in)) != PGAMD_OK) return rc;
+      HIP_TRY(hipEventRecord(c->slice_ev[1 + 2 * i], in));
+      HIP_TRY(hipStreamWaitEvent(st, c->slice_ev[1 + 2 * i], 0));
+      if ((rc = solve(f, n, st)) != PGAMD_OK) return rc;
+      HIP_TRY(hipEventRecord(c->slice_ev[2 + 2 * i], st));
+    }
+    for (int i = 0; i < ns; i++) {   // after the loop: a copy to pageable memory holds the host until it is done
+      const size_t f = at[i], n = at[i + 1] - f;
+      HIP_TRY(hipStreamWaitEvent(out, c->slice_ev[2 + 2 * i], 0));
+      if ((rc = copy_out(f, n, out)) != PGAMD_OK) return rc;
+    }
+    if ((rc = copy_stats(0, npatch, st)) != PGAMD_OK) return rc;
+    HIP_TRY(hipEventRecord(c->slice_ev[0], out));
+    HIP_TRY(hipStreamWaitEvent(st, c->slice_ev[0], 0));
+    c->last_npatch = poisson ? npatch : 0;
+    return PGAMD_OK;
+  }
+  for (int s = 0; s < gpu_nstream; s++) {  // a. host -> device
+    if (count[s] > 0 && (rc = copy_in(first[s], count[s], c->streams[s])) != PGAMD_OK) return rc;
   }
   for (int s = 0; s < gpu_nstream; s++) {  // b. kernels
-    if (count[s] == 0) continue;
-    const size_t f = first[s];
-    rc = pgamd::enqueue_solve(c, c->d_rho + f * c->rho_n, c->d_pot_in + f * c->cpot_n, nullptr,
-                              c->d_pot_out + f * c->out_n, graacc ? c->d_flu + f * flu_n : nullptr, count[s], a, p,
-                              c->d_iters + f, c->d_status + f, c->streams[s]);
-    if (rc != PGAMD_OK) return rc;
+    if (count[s] > 0 && (rc = solve(first[s], count[s], c->streams[s])) != PGAMD_OK) return rc;
   }
   for (int s = 0; s < gpu_nstream; s++) {  // c. device -> host
     if (count[s] == 0) continue;
-    hipStream_t st = c->streams[s];
-    const size_t f = first[s], n = count[s];
-    if (poisson) {
-      HIP_TRY(hipMemcpyAsync(h_pot_out + f * c->out_n, c->d_pot_out + f * c->out_n, n * c->out_n * 4,
-                             hipMemcpyDeviceToHost, st));
-      HIP_TRY(hipMemcpyAsync(c->h_iters + f, c->d_iters + f, n * 4, hipMemcpyDeviceToHost, st));
-      HIP_TRY(hipMemcpyAsync(c->h_status + f, c->d_status + f, n * 4, hipMemcpyDeviceToHost, st));
-    }
-    if (graacc)
-      HIP_TRY(hipMemcpyAsync(h_flu + f * flu_n, c->d_flu + f * flu_n, n * flu_n * 4, hipMemcpyDeviceToHost, st));
+    if ((rc = copy_out(first[s], count[s], c->streams[s])) != PGAMD_OK) return rc;
+    if ((rc = copy_stats(first[s], count[s], c->streams[s])) != PGAMD_OK) return rc;
   }
   c->last_npatch = poisson ? npatch : 0;
   return PGAMD_OK;
@@ -389,6 +468,8 @@ int pgamd_synchronize(pgamd_context* c) {
   if (!c) return fail(PGAMD_ERR_ARG, "null context");
   HIP_TRY(hipSetDevice(c->device));
   for (auto s : c->streams) HIP_TRY(hipStreamSynchronize(s));
+  for (auto s : c->copy)   // joined to the streams above, but not by a call that failed half-way
+    if (s) HIP_TRY(hipStreamSynchronize(s));
   return PGAMD_OK;
 }
 
