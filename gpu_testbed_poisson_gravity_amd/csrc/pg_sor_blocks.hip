@@ -18,6 +18,11 @@
 // in the other colour), the Dirichlet layer included.  A cell update costs two LDS reads (across the x pair and the y
 // pair), one more at the ends of a chunk of planes, and one write.  HP and PL were chosen for the fewest bank conflicts of
 // 32 lanes per cycle (FP32) or 16 (FP64): none at ghost sizes 1 and 5.
+// FP64 at ghost size 5 keeps a column's cells of one colour together instead, so that the two cells of a thread's column
+// are one 16-byte read or write (BlockGeo::PAIRS): 64 lanes in 4 cycles, as an 8-byte read.  It was bound by the LDS (70%
+// busy, VALU 64%); now the LDS is busy for half of the time and the VALU for 62%, and what is left is their latency with
+// three patches (12 waves) per CU.  MI355X, 4096 patches to a relative residual of 1e-10: 1148 -> 1055 us; with 10 words per
+// column and rows shifted in turn (writes with two-way conflicts) 1113 us.
 //
 // The one-wavefront kernel decides where to stop on FP32 sums in its own order.  The FP32 form here must stop at the same
 // iteration: it compares sums reduced as a tree over the workgroup, and where the two sides are within 2e-5 of each other
@@ -49,8 +54,14 @@ struct BlockGeo {
   static constexpr bool F64 = sizeof(T) == 8;
   static constexpr int HP = N / 2 + (GS == 1 || GS == 4 || (GS == 5 && !F64) ? 1 : 0);
   static constexpr int PL = N * HP + (GS == 1 && !F64 ? 12 : GS == 2 ? (F64 ? 3 : 1) : GS == 4 && F64 ? 2 : 0);
-  static constexpr bool XMAJOR = GS >= 3;                 // lane order within a plane: x blocks slow
-  static constexpr int CS = N * PL;                       // words per colour
+  // Pairs: a column's interior cells of one colour lie together, so that a thread's two are one 16-byte word; x pairs of
+  // columns are XP words apart (their two Dirichlet cells last), rows RP.  A 16-byte read serves lanes 0-3, 12-15 and 20-27 of
+  // 32 in a cycle, then the others; a write 8 lanes of 32 banks: XP is 2 modulo 16 and RP 8 modulo 16, without conflicts.
+  static constexpr bool PAIRS = F64 && GS == 5 && PLANES == 4;
+  static constexpr int XP = R + 2, RP = (N / 2 * XP + 7) / 16 * 16 + 8;
+  static_assert(!PAIRS || (XP % 16 == 2 && RP >= N / 2 * XP), "bank-free");
+  static constexpr bool XMAJOR = GS >= 3 && !PAIRS;       // lane order within a plane: x blocks slow
+  static constexpr int CS = PAIRS ? N * RP : N * PL;      // words per colour
   static constexpr int NC = C - 2;                        // coarse cells with children in the cube, per axis
   static constexpr int ROWS = THREADS / 16;
   static constexpr int RED = 2 * CS;                      // two pairs of row sums
@@ -61,7 +72,12 @@ struct BlockGeo {
   __device__ static bool edge(int x, int y, int z) {
     return (x == 0 || x == N - 1) + (y == 0 || y == N - 1) + (z == 0 || z == N - 1) > 1;
   }
-  __device__ static int word(int x, int y, int z) { return ((x + y + z) & 1) * CS + z * PL + y * HP + (x >> 1); }
+  __device__ static int column(int x, int y) { return y * RP + (x >> 1) * XP + (x & 1) * (R / 2); }
+  __device__ static int word(int x, int y, int z) {
+    const int c = ((x + y + z) & 1) * CS;
+    if (PAIRS) return z == 0 || z == N - 1 ? c + y * RP + (x >> 1) * XP + R + (x & 1) : c + column(x, y) + ((z - 1) >> 1);
+    return c + z * PL + y * HP + (x >> 1);
+  }
 };
 
 // A thread's cells.
@@ -71,7 +87,9 @@ struct Block {
   static constexpr int H = G::H;
   T phi[2][2][H], cr[2][2][H];   // [yy][xx][zi]; cr = Const*rho
   int x0, y0, z0;                // cube coordinates of the first cell, all odd
+  static constexpr int kX1 = G::XP - G::R / 2;   // pairs: words from the first column of a block to the second
   int own;                       // word of (x0, y0, z0) without its colour
+  int below[2], above[2];        // pairs: offsets of the words below and above the chunk in a column
   int chunk, column;             // chunk of planes; lane of the column in the one-wavefront kernel
   bool active;
 
@@ -84,11 +102,23 @@ struct Block {
     x0 = 2 * m + 1;
     y0 = 2 * yb + 1;
     z0 = chunk * H + 1;
-    own = z0 * G::PL + y0 * G::HP + m;
+    if (G::PAIRS) {
+      static_assert(!G::PAIRS || (H == 4 && G::OWNERS == G::THREADS), "two cells of each colour per column");
+      own = G::column(x0, y0) + 2 * chunk;
+#pragma unroll
+      for (int xx = 0; xx < 2; xx++) {
+        const int end = xx ? G::R : G::R / 2 + 1;   // the column's Dirichlet cell
+        below[xx] = chunk ? -1 : end;
+        above[xx] = chunk < G::CHUNKS - 1 ? 2 : end - 2 * chunk;
+      }
+    } else {
+      own = z0 * G::PL + y0 * G::HP + m;
+    }
     column = GS >= 4 ? m * G::MX + yb : yb * G::MX + m;
   }
   static constexpr int xx_of(int c, int yy, int zi) { return (c + yy + zi + 1) & 1; }
   __device__ __forceinline__ int word(int c, int yy, int xx, int zi) const {
+    if (G::PAIRS) return own + c * G::CS + yy * G::RP + xx * kX1 + (zi >> 1);
     return own + c * G::CS + zi * G::PL + yy * G::HP + xx;
   }
   // Residual of the cell of colour c at (yy, zi), reference operand order (CPU_PoissonSolver_SOR.cpp:247-250).
@@ -103,10 +133,37 @@ struct Block {
     const T ip = xx == 0 ? phi[yy][1][zi] : io, im = xx == 1 ? phi[yy][0][zi] : io;
     return kp + km + jp + jm + ip + im - T(6) * phi[yy][xx][zi] - cr[yy][xx][zi];
   }
+  // Pairs: residuals of colour c in column (yy, xx), r[2 zi + yy].
+  template <int c, int yy, int xx>
+  __device__ __forceinline__ void column_residuals(const T* __restrict__ lds, T (&r)[2 * H]) const {
+    constexpr int zs = (c + 1 + yy + xx) & 1, b = (1 - c) * G::CS;
+    const int o = own + b + yy * G::RP + xx * kX1;
+    struct alignas(16) Two { T v[2]; };
+    const Two io = *reinterpret_cast<const Two*>(lds + o + (xx ? G::R / 2 : -G::R / 2));
+    const Two jo = *reinterpret_cast<const Two*>(lds + o + (yy ? G::RP : -G::RP));
+    const T end = lds[o + (zs ? above[xx] : below[xx])];
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+      const int zi = zs + 2 * u;
+      const T kp = zi + 1 < H ? phi[yy][xx][zi + 1 < H ? zi + 1 : 0] : end;
+      const T km = zi > 0 ? phi[yy][xx][zi > 0 ? zi - 1 : 0] : end;
+      const T jp = yy == 0 ? phi[1][xx][zi] : jo.v[u], jm = yy == 1 ? phi[0][xx][zi] : jo.v[u];
+      const T ip = xx == 0 ? phi[yy][1][zi] : io.v[u], im = xx == 1 ? phi[yy][0][zi] : io.v[u];
+      r[2 * zi + yy] = kp + km + jp + jm + ip + im - T(6) * phi[yy][xx][zi] - cr[yy][xx][zi];
+    }
+  }
   // f(q, yy, xx, zi, residual) for every cell of colour c, q = 2 zi + yy
   template <int c, int q = 0, class F>
   __device__ __forceinline__ void each(const T* __restrict__ lds, F f) const {
-    if constexpr (q < 2 * H) {
+    if constexpr (G::PAIRS) {
+      T r[2 * H];
+      column_residuals<c, 0, 0>(lds, r);
+      column_residuals<c, 0, 1>(lds, r);
+      column_residuals<c, 1, 0>(lds, r);
+      column_residuals<c, 1, 1>(lds, r);
+#pragma unroll
+      for (int i = 0; i < 2 * H; i++) f(i, i & 1, xx_of(c, i & 1, i >> 1), i >> 1, r[i]);
+    } else if constexpr (q < 2 * H) {
       const T r = residual<c, (q & 1), (q >> 1)>(lds);
       f(q, q & 1, xx_of(c, q & 1, q >> 1), q >> 1, r);
       each<c, q + 1>(lds, f);
@@ -114,7 +171,16 @@ struct Block {
   }
   template <int c>
   __device__ __forceinline__ void publish(T* __restrict__ lds) const {
-    if (active) {
+    if (G::PAIRS) {   // every thread owns a block
+      struct alignas(16) Two { T v[2]; };
+#pragma unroll
+      for (int yy = 0; yy < 2; yy++)
+#pragma unroll
+        for (int xx = 0; xx < 2; xx++) {
+          const int zs = (c + 1 + yy + xx) & 1;
+          *reinterpret_cast<Two*>(lds + word(c, yy, xx, 0)) = Two{{phi[yy][xx][zs], phi[yy][xx][zs + 2 < H ? zs + 2 : 0]}};
+        }
+    } else if (active) {
 #pragma unroll
       for (int zi = 0; zi < H; zi++)
 #pragma unroll
@@ -627,21 +693,27 @@ hipError_t launch_tasks_as(const MixedBatch& b, const SolveParams& p, int ppw, i
   return hipGetLastError();
 }
 
-// Two planes per thread instead of four at ghost sizes 3 and 5: twice the waves per patch, for batches that leave the GPU
-// short of them.  MI355X, us per call with 4 / 2 planes (interpolated start, FP32 stall rule; FP64 to 1e-10): GS 3, 8
-// patches 49 / 35, 1024: 61 / 55, 1536: 76 / 74, 2048: 84 / 101; GS 5, 8: 61 / 45, 512: 76 / 66, 768: 85 / 83, 1024: 96 / 116.
-// FP64 GS 3, 8: 122 / 97, 512: 160 / 140, 4096: 639 / 741; GS 5, 256: 154 / 140, 512: 197 / 208.
-bool two_planes(int gs, bool f64, int npatch) { return npatch <= (gs == 3 ? (f64 ? 512 : 1024) : (f64 ? 256 : 512)); }
+// Two planes per thread instead of four at ghost sizes 3 and 5 (FP32 only: FP64 has the paired layout for four): twice the
+// waves per patch, for batches that leave the GPU short of them.  MI355X, us per call with 4 / 2 planes (interpolated start,
+// FP32 stall rule; FP64 to 1e-10): GS 3, 8 patches 49 / 35, 1024: 61 / 55, 1536: 76 / 74, 2048: 84 / 101; GS 5, 8: 61 / 45,
+// 512: 76 / 66, 768: 85 / 83, 1024: 96 / 116.  FP64 GS 3, 8: 122 / 97, 512: 160 / 140, 4096: 639 / 741; GS 5, 8: 122 / 124,
+// 256: 140 / 144, 512: 185 / 214, 4096: 1004 / 1250.
+bool two_planes(int gs, bool f64, int npatch) { return npatch <= (gs == 3 ? (f64 ? 512 : 1024) : (f64 ? 0 : 512)); }
 
 template <typename PT>
 hipError_t launch_blocks(const UniformBatchT<typename PT::real>& b, const PT& p, bool wave_dpp, hipStream_t s) {
-  const bool two = two_planes(b.gs, sizeof(typename PT::real) == 8, b.npatch);
+  constexpr bool F64 = sizeof(typename PT::real) == 8;
+  const bool two = two_planes(b.gs, F64, b.npatch);
   switch (b.gs) {
     case 1: return launch_as<1, 2>(b, p, wave_dpp, s);
     case 2: return launch_as<2, 2>(b, p, wave_dpp, s);
     case 3: return two ? launch_as<3, 2>(b, p, wave_dpp, s) : launch_as<3, 4>(b, p, wave_dpp, s);
     case 4: return launch_as<4, 2>(b, p, wave_dpp, s);
-    case 5: return two ? launch_as<5, 2>(b, p, wave_dpp, s) : launch_as<5, 4>(b, p, wave_dpp, s);
+    case 5:
+      if constexpr (!F64) {
+        if (two) return launch_as<5, 2>(b, p, wave_dpp, s);
+      }
+      return launch_as<5, 4>(b, p, wave_dpp, s);
   }
   return hipErrorInvalidValue;
 }
