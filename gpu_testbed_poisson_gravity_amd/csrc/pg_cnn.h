@@ -29,7 +29,7 @@ constexpr int kCnnOutputs = kCnnVox * kCnnOut;               // fp32 values per 
 hipError_t cnn_conv_fwd(const uint16_t* X, const uint16_t* W, const float* b, uint16_t* Y, float* D, int n, int mode,
                         hipStream_t s);
 // Forward, loss against T [n][8^3][8] (squared error, plus res_weight times the squared residual it leaves) and output
-// gradients: y[1..5] (borders untouched), dH [6][n][8^3][16] and cnn_train_blocks(n) loss partials (sums).
+// gradients: y[1..5] (borders untouched), dH [6][n][8^3][16] and cnn_train_blocks(n) loss partials (sums, in pinned host memory).
 constexpr int kCnnTrainBlocks = 256;   // one per CU
 int cnn_train_blocks(int n);
 hipError_t cnn_train_pass(const uint16_t* x0, const uint16_t* WL, const uint16_t* WT, const float* P, const float* T,

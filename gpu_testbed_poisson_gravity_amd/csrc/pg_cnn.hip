@@ -206,7 +206,7 @@ static_assert(sizeof(TrainLds) <= 160 * 1024 && sizeof(TrainLds) % 16 == 0, "one
 struct TrainOut {
   u16* y[kCnnLayers];   // y[1..5]: layer outputs, padded [n][10^3][16]
   u16* dh;              // [6][n][8^3][16]
-  float* loss;          // one partial per workgroup
+  float* loss;          // one partial per workgroup, host memory
 };
 
 // A value the compiler cannot see through: addresses derived from it are computed in each phase, not kept across them.
@@ -462,7 +462,7 @@ __global__ void __launch_bounds__(kTrainThreads, kTrainThreads / 256) train_pass
   if (threadIdx.x == 0) {
     float sum = lds.red[0];
     for (int i = 1; i < kTrainThreads / 64; i++) sum += lds.red[i];
-    out.loss[blockIdx.x] = sum;
+    __hip_atomic_store(out.loss + blockIdx.x, sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }
 

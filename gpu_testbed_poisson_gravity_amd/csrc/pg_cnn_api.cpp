@@ -38,6 +38,7 @@ struct pgamd_cnn {
   int step = 0;
   float res_weight = 0.0f;  // weight of the residual term of the loss (pgamd_cnn_set_loss)
   float *p = nullptr, *g = nullptr, *m = nullptr, *v = nullptr;
+  float* lossp = nullptr;   // loss partials [kCnnTrainBlocks], pinned host memory
   uint16_t* wb = nullptr;   // BF16 W1..W6 in the forward layout [16][480]
   uint16_t* wt = nullptr;   // BF16 W1..W6 transposed, taps reversed, lane-major (input gradients)
   uint16_t* wl = nullptr;   // BF16 W1..W6 forward layout, lane-major (the fused kernels)
@@ -46,7 +47,7 @@ struct pgamd_cnn {
   bool train_ws = false;
   uint16_t* y[6] = {};      // y1..y5, padded [n][10^3][16] with zero borders (y[0] unused: the input)
   uint16_t* dh = nullptr;   // output gradients of the six layers, [6][n][8^3][16]
-  float *d = nullptr, *part = nullptr, *lossp = nullptr;
+  float *d = nullptr, *part = nullptr;
   // pipelined warm-start solve: fork event and one event per chunk
   hipEvent_t ev[kMaxChunks + 1] = {};
 };
@@ -61,9 +62,8 @@ void free_ws(pgamd_cnn* n) {
   hipFree(n->dh);
   hipFree(n->d);
   hipFree(n->part);
-  hipFree(n->lossp);
   n->dh = nullptr;
-  n->d = n->part = n->lossp = nullptr;
+  n->d = n->part = nullptr;
   n->cap = 0;
   n->train_ws = false;
 }
@@ -83,7 +83,6 @@ int ensure_ws(pgamd_cnn* n, int count, bool train) {
   if (train) {
     ok &= hipMalloc(&n->dh, kCnnLayers * act * 2) == hipSuccess;
     ok &= hipMalloc(&n->part, (size_t)kCnnLayers * cnn_grad_parts(count) * kCnnLayerParams * 4) == hipSuccess;
-    ok &= hipMalloc(&n->lossp, cnn_train_blocks(count) * 4) == hipSuccess;
   }
   if (!ok) {
     free_ws(n);
@@ -115,23 +114,21 @@ int forward(pgamd_cnn* n, const uint16_t* x0, int count, hipStream_t s) {
   return PGAMD_OK;
 }
 
-// Forward + backward; gradients (mean squared error, plus the residual term when res_weight > 0) go to n->g,
+// Forward + backward; gradients (mean squared error, plus the residual term when res_weight > 0) go to g,
 // loss partials to lossp.
-int forward_backward(pgamd_cnn* n, const uint16_t* x0, const float* target, int count, hipStream_t s) {
+int forward_backward(pgamd_cnn* n, const uint16_t* x0, const float* target, int count, float* g, hipStream_t s) {
   CK(cnn_train_pass(x0, n->wl, n->wt, n->p, target, n->y, n->dh, n->lossp, count, n->res_weight, s));
   const uint16_t* x[kCnnLayers] = {x0, n->y[1], n->y[2], n->y[3], n->y[4], n->y[5]};
-  CK(cnn_weight_grad(x, n->dh, count, n->part, n->g, s));
+  CK(cnn_weight_grad(x, n->dh, count, n->part, g, s));
   return PGAMD_OK;
 }
 
+// The loss, once the stream has run: the partials are in host memory.
 float read_loss(pgamd_cnn* n, int count, hipStream_t s) {
-  float h[kCnnTrainBlocks];
+  if (hipStreamSynchronize(s) != hipSuccess) return NAN;
   const int parts = cnn_train_blocks(count);
-  if (hipMemcpyAsync(h, n->lossp, parts * sizeof(float), hipMemcpyDeviceToHost, s) != hipSuccess ||
-      hipStreamSynchronize(s) != hipSuccess)
-    return NAN;
   double t = 0.0;
-  for (int i = 0; i < parts; i++) t += h[i];
+  for (int i = 0; i < parts; i++) t += n->lossp[i];
   return (float)(t / ((double)count * kCnnOutputs));
 }
 
@@ -163,7 +160,8 @@ int pgamd_cnn_create(pgamd_context* ctx, uint64_t seed, pgamd_cnn** out) {
   if (hipSetDevice(n->device) != hipSuccess || hipMalloc(&n->p, kCnnParams * 4) != hipSuccess ||
       hipMalloc(&n->g, kCnnParams * 4) != hipSuccess || hipMalloc(&n->m, kCnnParams * 4) != hipSuccess ||
       hipMalloc(&n->v, kCnnParams * 4) != hipSuccess || hipMalloc(&n->wb, kCnnLayers * kWF * 2) != hipSuccess ||
-      hipMalloc(&n->wt, kCnnLayers * kWF * 2) != hipSuccess || hipMalloc(&n->wl, kCnnLayers * kWF * 2) != hipSuccess) {
+      hipMalloc(&n->wt, kCnnLayers * kWF * 2) != hipSuccess || hipMalloc(&n->wl, kCnnLayers * kWF * 2) != hipSuccess ||
+      hipHostMalloc((void**)&n->lossp, kCnnTrainBlocks * 4) != hipSuccess) {
     pgamd_cnn_destroy(n);
     return set_error(PGAMD_ERR_NOMEM, "CNN parameter allocation failed");
   }
@@ -202,6 +200,7 @@ int pgamd_cnn_destroy(pgamd_cnn* n) {
   hipFree(n->wb);
   hipFree(n->wt);
   hipFree(n->wl);
+  hipHostFree(n->lossp);
   for (hipEvent_t e : n->ev)
     if (e) hipEventDestroy(e);
   delete n;
@@ -246,9 +245,8 @@ int pgamd_cnn_loss_grad(pgamd_cnn* n, const uint16_t* d_x0, const float* d_targe
   hipStream_t s = (hipStream_t)stream;
   int rc = ensure_ws(n, count, true);
   if (rc != PGAMD_OK) return rc;
-  rc = forward_backward(n, d_x0, d_target, count, s);
+  rc = forward_backward(n, d_x0, d_target, count, d_grad ? d_grad : n->g, s);
   if (rc != PGAMD_OK) return rc;
-  if (d_grad) CK(hipMemcpyAsync(d_grad, n->g, kCnnParams * 4, hipMemcpyDeviceToDevice, s));
   if (loss) *loss = read_loss(n, count, s);
   return PGAMD_OK;
 }
@@ -260,7 +258,7 @@ int pgamd_cnn_train_step(pgamd_cnn* n, const uint16_t* d_x0, const float* d_targ
   hipStream_t s = (hipStream_t)stream;
   int rc = ensure_ws(n, count, true);
   if (rc != PGAMD_OK) return rc;
-  rc = forward_backward(n, d_x0, d_target, count, s);
+  rc = forward_backward(n, d_x0, d_target, count, n->g, s);
   if (rc != PGAMD_OK) return rc;
   n->step++;
   const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
