@@ -607,7 +607,7 @@ def main():
         fp64 = {"value": a.npatch / (ms64 * 1e-3), "ms_per_step": ms64, "mean_iters": float(it64.mean()),
                 "iters_sum": float(it64.astype(np.float64).sum()),
                 "converged": int(((d_st.cpu().numpy() & pg.STATUS_CONVERGED) != 0).sum()), "steps": steps64,
-                "note": "sor64_kernel, zero guess to relative residual 1e-5 in FP64; the plain leg in FP64"}
+                "note": "sor_blocks_kernel, zero guess to relative residual 1e-5 in FP64; the plain leg in FP64"}
         log(f"[bench] fp64 plain: {fp64['value']:.4g} patch-solves/s, {fp64['mean_iters']:.1f} iterations")
         del r64, c64, f64, fl64, o64
     net = None
@@ -638,10 +638,10 @@ def main():
         roofs["sor_interp"] = lds_roof(interp, "interp")
     if fp64 is not None:
         ops64 = fp64["iters_sum"] * R ** 3 * VALU_OPS_PER_UPDATE
-        roofs["sor64"] = {"kernel": "sor64_kernel", "bound": "valu", "achieved": ops64 / (fp64["ms_per_step"] * 1e-3) / 1e12,
+        roofs["sor64"] = {"kernel": "sor_blocks_kernel", "bound": "valu", "achieved": ops64 / (fp64["ms_per_step"] * 1e-3) / 1e12,
                           "peak": VALU_PEAK / 1e12, "unit": "Tops/s (FP64)",
                           "frac": ops64 / (fp64["ms_per_step"] * 1e-3) / VALU_PEAK,
-                          "traffic": traffic.get(("sor64_kernel", "fp64")), "launch_ms": fp64["ms_per_step"]}
+                          "traffic": traffic.get(("sor_blocks_kernel", "fp64")), "launch_ms": fp64["ms_per_step"]}
     roof = roof_sor
     if warm_serial is not None:
         flop = CNN_USEFUL_FLOP * a.npatch

@@ -48,7 +48,8 @@ constexpr MgLevels mg_levels_of(int n0) {
 // 0 and keeps those cells' solution and right-hand side in registers; LDS serves the neighbours outside the block.
 // H is even, so that which of a block's cells has which colour does not depend on the thread, and divides R:
 // H = 4 where that fills the waves (GS 3: 108 of 128 threads, GS 5: 256), else 2 (GS 1: 64, GS 2: 125 of 128,
-// GS 4: 343 of 384).  A cell of a coarser level (at most 7^3) belongs to one thread, two neighbours along x each.
+// GS 4: 343 of 384).  A cell of a coarser level belongs to one thread, two neighbours along x where the level has more
+// cells than the workgroup threads (mg_coarse_cells).
 //
 // Level-0 layout in LDS: colour c = (x+y+z)&1, plane z, then the plane's cells of that colour as
 // [y parity][y/2][x/2] (interior coordinates), so consecutive threads touch consecutive words; then the plane's
@@ -925,8 +926,9 @@ size_t lds_bytes_mg(int gs) {
 }
 
 // Largest batch for mg_patch_cells.  Measured on MI355X, us per call (interpolated start, 3+3 smoothing; FP32 to 1e-5,
-// FP64 to 1e-10), mg_patch / mg_patch_cells: FP32 GS 1, 512 patches 33 / 20, 1024: 35 / 26 (its limit: four workgroups
-// per CU); GS 2, 512: 31 / 28 (two per CU).  FP64 GS 1, 512: 73 / 53; GS 2, 256: 72 / 60 (one per CU), 512: 79 / 99.
+// FP64 to 1e-10), mg_patch / mg_patch_cells: FP32 GS 1, 512 patches 31 / 20, 1024: 32 / 26 (its limit: four workgroups
+// per CU), 1536: 38 / 37; GS 2, 256: 26 / 21, 512: 28.0 / 27.7 (two per CU), 1024: 31 / 43.  FP64 GS 1, 512: 64 / 52,
+// 1024: 71 / 101; GS 2, 256: 63 / 59 (one per CU), 512: 74 / 108.
 static bool mg_small(int gs, size_t word, int n) {
   if (gs == 1) return n <= (word == 8 ? 512 : 1024);
   return gs == 2 && n <= (word == 8 ? 256 : 512);
