@@ -26,15 +26,19 @@ __device__ __forceinline__ T row_sum(T v) {
   return v + dpp<0x140>(v);   // row mirror
 }
 
+__device__ __forceinline__ float lane_value(float v, int lane) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
+}
+__device__ __forceinline__ double lane_value(double v, int lane) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane), __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+
 // Sum over the wavefront: rows of 16 lanes as above, then (r0 + r1) + (r2 + r3) from scalar registers, so every lane gets
 // the same bits.
-__device__ __forceinline__ float wave_sum_dpp(float v) {
+template <typename T>
+__device__ __forceinline__ T wave_sum_dpp(T v) {
   v = row_sum(v);
-  const float r0 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 0));
-  const float r1 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 16));
-  const float r2 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 32));
-  const float r3 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 48));
-  return (r0 + r1) + (r2 + r3);
+  return (lane_value(v, 0) + lane_value(v, 16)) + (lane_value(v, 32) + lane_value(v, 48));
 }
 
 // Butterfly sum over the wavefront (partners 32, 16, ... 1 apart); with lanes beyond a shorter segment at zero, the bits

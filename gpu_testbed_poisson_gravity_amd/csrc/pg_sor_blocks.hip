@@ -63,9 +63,9 @@ struct BlockGeo {
   static constexpr bool XMAJOR = GS >= 3 && !PAIRS;       // lane order within a plane: x blocks slow
   static constexpr int CS = PAIRS ? N * RP : N * PL;      // words per colour
   static constexpr int NC = C - 2;                        // coarse cells with children in the cube, per axis
-  static constexpr int ROWS = THREADS / 16;
-  static constexpr int RED = 2 * CS;                      // two pairs of row sums
-  static constexpr int SCRATCH = RED + 4 * ROWS;          // FP32: 2H values per column (ordered sums), one result
+  static constexpr int WAVES = THREADS / 64;
+  static constexpr int RED = 2 * CS;                      // two pairs of wave sums
+  static constexpr int SCRATCH = RED + 4 * WAVES;         // FP32: 2H values per column (ordered sums), one result
   static constexpr int WORDS = SCRATCH + (F64 ? 0 : 2 * H * 64 + 1);
   static_assert(C * C * C <= 2 * CS, "the coarse potential fits where the cube goes");
   // cube cell on two or three faces
@@ -313,24 +313,37 @@ __device__ __forceinline__ void blocks_interpolate_odd(Block<GS, T, PLANES>& o, 
   }
 }
 
+// Sum of the waves' values (one wave: each lane has it).
+template <int N, typename T>
+__device__ __forceinline__ T blocks_total(const T* red) {
+  if constexpr (N == 1)
+    return red[0];
+  else
+    return blocks_total<N / 2>(red) + blocks_total<N - N / 2>(red + N / 2);
+}
+template <int WAVES, typename T>
+__device__ __forceinline__ void blocks_put(T wave, T* red) {
+  if (WAVES > 1 && (threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = wave;
+}
+template <int WAVES, typename T>
+__device__ __forceinline__ T blocks_get(T wave, const T* red) {
+  if constexpr (WAVES == 1)
+    return wave;
+  else
+    return blocks_total<WAVES>(red);
+}
+
 // Sums of a and b over the workgroup, the same bits in every thread.  No barrier afterwards: the next use of the same
 // `red` comes after at least one other barrier.
-template <int ROWS, typename T>
+template <int WAVES, typename T>
 __device__ __forceinline__ void blocks_sum2(T& a, T& b, T* red) {
-  a = row_sum(a);
-  b = row_sum(b);
-  if ((threadIdx.x & 15) == 0) {
-    red[threadIdx.x >> 4] = a;
-    red[ROWS + (threadIdx.x >> 4)] = b;
-  }
+  a = wave_sum_dpp(a);
+  b = wave_sum_dpp(b);
+  blocks_put<WAVES>(a, red);
+  blocks_put<WAVES>(b, red + WAVES);
   __syncthreads();
-  a = red[0];
-  b = red[ROWS];
-#pragma unroll
-  for (int k = 1; k < ROWS; k++) {
-    a += red[k];
-    b += red[ROWS + k];
-  }
+  a = blocks_get<WAVES>(a, red);
+  b = blocks_get<WAVES>(b, red + WAVES);
 }
 
 // The sums of the one-wavefront kernel (FP32): per column, the cells of a colour from the bottom up, lane `column` of the
@@ -481,7 +494,7 @@ __device__ __forceinline__ void blocks_patch(T* __restrict__ lds, const T* __res
     o.template each<0>(lds, [&](int q, int, int, int, T r) { num += fabs(black[q] = r); });
     o.cells([&](int yy, int xx, int zi) { den += fabs(o.phi[yy][xx][zi]); });
     if (!o.active) num = den = T(0);
-    blocks_sum2<G::ROWS>(num, den, red);
+    blocks_sum2<G::WAVES>(num, den, red);
     bool keep = num <= P.guess_tol * den;
     if constexpr (ORDERED) {
       if (too_close(num, P.guess_tol * den)) {
@@ -518,7 +531,7 @@ __device__ __forceinline__ void blocks_patch(T* __restrict__ lds, const T* __res
       o.cells([&](int yy, int xx, int zi) { den += fabs(o.phi[yy][xx][zi]); });
       num = num + P.damp * black_sum;
       if (!o.active) num = den = T(0);
-      blocks_sum2<G::ROWS>(num, den, red);
+      blocks_sum2<G::WAVES>(num, den, red);
       bool stop = num <= P.rel_tol * den;
       if constexpr (ORDERED) {
         if (too_close(num, P.rel_tol * den)) {
@@ -562,13 +575,11 @@ __device__ __forceinline__ void blocks_patch(T* __restrict__ lds, const T* __res
     o.template publish<0>(lds);
     if (stall) {
       T tot = o.active ? sum + black_sum : T(0);
-      T* r2 = red + 2 * G::ROWS;
-      tot = row_sum(tot);
-      if ((t & 15) == 0) r2[t >> 4] = tot;
+      T* r2 = red + 2 * G::WAVES;
+      tot = wave_sum_dpp(tot);
+      blocks_put<G::WAVES>(tot, r2);
       __syncthreads();
-      tot = r2[0];
-#pragma unroll
-      for (int k = 1; k < G::ROWS; k++) tot += r2[k];
+      tot = blocks_get<G::WAVES>(tot, r2);
       if (it + 1 >= P.min_iter) {
         bool grew = tot > old;
         if constexpr (ORDERED) {
