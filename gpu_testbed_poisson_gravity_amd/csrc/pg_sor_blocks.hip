@@ -21,8 +21,8 @@
 // FP64 at ghost size 5 keeps a column's cells of one colour together instead, so that the two cells of a thread's column
 // are one 16-byte read or write (BlockGeo::PAIRS): 64 lanes in 4 cycles, as an 8-byte read.  It was bound by the LDS (70%
 // busy, VALU 64%); now the LDS is busy for half of the time and the VALU for 62%, and what is left is their latency with
-// three patches (12 waves) per CU.  MI355X, 4096 patches to a relative residual of 1e-10: 1148 -> 1055 us; with 10 words per
-// column and rows shifted in turn (writes with two-way conflicts) 1113 us.
+// three patches (12 waves) per CU.  MI355X, 4096 patches to a relative residual of 1e-10: 1148 -> 1055 us (1004 with wave
+// sums for the stopping test); with 10 words per column and rows shifted in turn (writes with two-way conflicts) 1113 us.
 //
 // The one-wavefront kernel decides where to stop on FP32 sums in its own order.  The FP32 form here must stop at the same
 // iteration: it compares sums reduced as a tree over the workgroup, and where the two sides are within 2e-5 of each other
@@ -704,12 +704,12 @@ hipError_t launch_tasks_as(const MixedBatch& b, const SolveParams& p, int ppw, i
   return hipGetLastError();
 }
 
-// Two planes per thread instead of four at ghost sizes 3 and 5 (FP32 only: FP64 has the paired layout for four): twice the
-// waves per patch, for batches that leave the GPU short of them.  MI355X, us per call with 4 / 2 planes (interpolated start,
-// FP32 stall rule; FP64 to 1e-10): GS 3, 8 patches 49 / 35, 1024: 61 / 55, 1536: 76 / 74, 2048: 84 / 101; GS 5, 8: 61 / 45,
-// 512: 76 / 66, 768: 85 / 83, 1024: 96 / 116.  FP64 GS 3, 8: 122 / 97, 512: 160 / 140, 4096: 639 / 741; GS 5, 8: 122 / 124,
-// 256: 140 / 144, 512: 185 / 214, 4096: 1004 / 1250.
-bool two_planes(int gs, bool f64, int npatch) { return npatch <= (gs == 3 ? (f64 ? 512 : 1024) : (f64 ? 0 : 512)); }
+// Two planes per thread instead of four at ghost sizes 3 and 5 (FP32 only at 5: FP64 has the paired layout for four): twice
+// the waves per patch, for batches that leave the GPU short of them.  MI355X, us per call with 4 / 2 planes (interpolated
+// start, FP32 stall rule; FP64 to 1e-10): GS 3, 8 patches 50 / 36, 1024: 62 / 54, 1536: 75 / 70, 2048: 82 / 96; GS 5, 8:
+// 59 / 42, 512: 76 / 63, 768: 84 / 74, 1024: 95 / 103.  FP64 GS 3, 8: 124 / 94, 512: 159 / 132, 1024: 190 / 205; GS 5, 8:
+// 122 / 124, 256: 140 / 144, 512: 185 / 214, 4096: 1004 / 1250.
+bool two_planes(int gs, bool f64, int npatch) { return npatch <= (gs == 3 ? (f64 ? 512 : 1536) : (f64 ? 0 : 768)); }
 
 template <typename PT>
 hipError_t launch_blocks(const UniformBatchT<typename PT::real>& b, const PT& p, bool wave_dpp, hipStream_t s) {
@@ -732,10 +732,10 @@ hipError_t launch_blocks(const UniformBatchT<typename PT::real>& b, const PT& p,
 }  // namespace
 
 // Where the block form is the faster one.  MI355X, us per call, one wavefront per patch (or group) / blocks, FP32 to 1e-5
-// from the interpolated start: GS 1, 8 patches 84 / 41, 4096: 107 / 69, 16384: 255 / 253; GS 2, 8: 84 / 39, 16384: 473 / 416
-// (25 of 32 lanes against 125 of 128); GS 3, 8: 88 / 43, 2048: 127 / 102, 16384: 832 / 658 (36 of 64 lanes against 108 of
-// 128); GS 4, 8: 95 / 46, 1024: 119 / 116, 1536: 131 / 165; GS 5, 8: 103 / 49, 1024: 133 / 96, 1536: 148 / 156 (the
-// one-wavefront kernel needs fewer reductions and reads once a launch fills the GPU).
+// from the interpolated start: GS 1, 8 patches 84 / 40, 4096: 109 / 69, 16384: 252 / 248; GS 2, 8: 83 / 39, 16384: 471 / 406
+// (25 of 32 lanes against 125 of 128); GS 3, 8: 87 / 43, 2048: 129 / 102, 16384: 821 / 633 (36 of 64 lanes against 108 of
+// 128); GS 4, 8: 95 / 43, 1024: 121 / 92, 1280: 124 / 124, 1536: 132 / 146; GS 5, 8: 103 / 44, 1024: 136 / 95, 1280:
+// 141 / 136, 1536: 148 / 150 (the one-wavefront kernel needs fewer reductions and reads once a launch fills the GPU).
 bool sor_blocks_better(int gs, int npatch) { return gs <= 3 || npatch <= 1024; }
 
 hipError_t launch_sor_blocks(const UniformBatch& b, const SolveParams& p, bool wave_dpp, hipStream_t s) {

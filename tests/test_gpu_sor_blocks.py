@@ -131,3 +131,10 @@ def test_fp64_forms_agree(gs, n):
     many = pg.solve_host_f64(rho[at], cpot[at], flu[at], **kw)
     for x, y in zip(few, many):
         assert np.array_equal(x[at], y)
+
+
+@pytest.mark.parametrize("gs, n", [(3, 1536), (3, 1537), (5, 768), (5, 769)])
+def test_blocks_match_at_plane_changes(gs, n):
+    """Batch sizes where the planes per thread change."""
+    _same(gs, n, dict(term_mode=pg.TERM_REFERENCE), pg.solver_args(sor_min_iter=10, sor_max_iter=60, sor_omega=1.65,
+                                                                   poi_coeff=POI, dt=0.5))
