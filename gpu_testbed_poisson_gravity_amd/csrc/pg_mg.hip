@@ -163,11 +163,12 @@ __device__ __forceinline__ void level_sync() {
   }
 }
 
-// Block-wide sums of two values in a fixed order (bitwise reproducible for a given launch shape): rows of 16 lanes by
-// DPP, then the row sums through LDS (shuffles over the wave would cross the LDS crossbar twelve times in a row).
-template <int THREADS, typename T>
+// Block-wide sums of two values over the first ROWS rows of 16 threads (the others have zeros), in an order that does not
+// depend on the workgroup's size: rows by DPP, then the row sums through LDS as a tree (shuffles over the wave would cross
+// the LDS crossbar twelve times in a row).
+template <int ROWS, typename T>
 __device__ __forceinline__ void block_sum2(T& a, T& b, T* red) {
-  constexpr int ROWS = THREADS / 16;
+  static_assert(ROWS <= kMgRows, "room for the row sums");
   a = row_sum(a);
   b = row_sum(b);
   const int w = threadIdx.x >> 4;
@@ -176,13 +177,8 @@ __device__ __forceinline__ void block_sum2(T& a, T& b, T* red) {
     red[kMgRows + w] = b;
   }
   __syncthreads();
-  a = red[0];
-  b = red[kMgRows];
-#pragma unroll
-  for (int k = 1; k < ROWS; k++) {
-    a += red[k];
-    b += red[kMgRows + k];
-  }
+  a = tree_sum<ROWS>(red);
+  b = tree_sum<ROWS>(red + kMgRows);
   __syncthreads();
 }
 
@@ -250,6 +246,27 @@ struct MgOwned {
       f(q & 1, xx_of(c, q & 1, q >> 1), q >> 1, nb);
       each_at<c, q + 1>(lds, f);
     }
+  }
+};
+
+// Sums of two values per cell over the patch, for the error estimate and the guess check.  At ghost sizes 1 and 2 the batch
+// size decides between mg_patch and mg_patch_cells (mg_small), and what a patch returns must not: both add in the order of
+// mg_patch_cells, whose threads hold an x pair each, four consecutive ones to a block of mg_patch.  The cells of a pair come
+// first (colour 0, then 1), then the pairs of a block by y and z, then the blocks as a tree over the threads.
+template <int GS, typename T>
+struct MgSums {
+  static constexpr bool PAIRS = GS <= 2;
+  static constexpr int NP = PAIRS ? 2 * MgGeo<GS>::H : 1;
+  T a[NP] = {}, b[NP] = {};
+  __device__ __forceinline__ void add(int yy, int zi, T va, T vb) {
+    const int q = PAIRS ? 2 * zi + yy : 0;
+    a[q] += va;
+    b[q] += vb;
+  }
+  __device__ __forceinline__ void total(bool active, T& sa, T& sb, T* red) const {
+    sa = active ? tree_sum<NP>(a) : T(0);
+    sb = active ? tree_sum<NP>(b) : T(0);
+    block_sum2<MgGeo<GS>::THREADS / 16>(sa, sb, red);
   }
 };
 
@@ -602,16 +619,15 @@ __device__ void mg_patch(T* __restrict__ lds, const T* __restrict__ rho, const T
   // as the SOR kernel does, and report it in the status.
   bool fell_back = false;
   if (P.init_mode >= 2 && P.guess_tol > T(0)) {
-    T num = T(0), den = T(0);
+    MgSums<GS, T> a;
     auto add = [&](int yy, int xx, int zi, T nb) {
       const int gi = ((o.z0 - 1 + zi) * R + (o.y0 - 1 + yy)) * R + (o.x0 - 1 + xx);
-      num += fabs(nb - T(6) * o.phi[yy][xx][zi] - P.cst * rho[gi]);
-      den += fabs(o.phi[yy][xx][zi]);
+      a.add(yy, zi, fabs(nb - T(6) * o.phi[yy][xx][zi] - P.cst * rho[gi]), fabs(o.phi[yy][xx][zi]));
     };
     o.template each<0>(lds, add);
     o.template each<1>(lds, add);
-    if (!o.active) num = den = T(0);
-    block_sum2<THREADS>(num, den, red);
+    T num, den;
+    a.total(o.active, num, den, red);
     fell_back = !(num <= P.guess_tol * den);
     if (fell_back) {
 #pragma unroll
@@ -667,15 +683,14 @@ __device__ void mg_patch(T* __restrict__ lds, const T* __restrict__ rho, const T
     if (P.mg_npost == 0) prolongate_level0<true>(o, lds);
     __syncthreads();
     for (int s = 0; s < P.mg_npost; s++) smooth_level0<GS>(o, lds, dh2);
-    T sd = T(0), ss = T(0);
+    MgSums<GS, T> a;
     auto sums = [&](int yy, int xx, int zi, T nb) {
-      sd += fabs(m_dh2 * (nb - T(6) * o.phi[yy][xx][zi]) + o.rhs[yy][xx][zi]);
-      ss += fabs(o.phi[yy][xx][zi]);
+      a.add(yy, zi, fabs(m_dh2 * (nb - T(6) * o.phi[yy][xx][zi]) + o.rhs[yy][xx][zi]), fabs(o.phi[yy][xx][zi]));
     };
     o.template each<0>(lds, sums);
     o.template each<1>(lds, sums);
-    if (!o.active) sd = ss = T(0);
-    block_sum2<THREADS>(sd, ss, red);
+    T sd, ss;
+    a.total(o.active, sd, ss, red);
     error = P.dh * P.dh * sd / ss;
     iter++;
   }
@@ -759,12 +774,15 @@ __device__ void mg_patch_cells(T* __restrict__ lds, const T* __restrict__ rho, c
   using M = MgGeo<GS>;
   constexpr int N = M::N, R = M::R, C = M::C, U = M::U, NC = C - 2, THREADS = mg_cell_threads(GS), LAST = R * R * R / 2 - 1;
   static_assert(LAST < THREADS && N * N * N <= 2 * M::CS && M::NLV >= 2, "one cell of each colour per thread");
+  static_assert(M::H == 2 && M::B.lpp == M::LP && THREADS == 4 * M::THREADS, "four threads to a block of mg_patch");
   T *sol = lds, *def = lds + M::FLOATS, *red = lds + M::off_red(), *stage = lds + 2 * M::CS;
   constexpr bool FRESH = sizeof(T) == 4;   // FP64 is compiled for fewer waves and keeps its weights in registers
   const int t = threadIdx.x;
   for (int q = t; q < M::STAGE; q += THREADS) stage[q] = cpot[q];
   const bool active = t <= LAST;
-  const int tc = active ? t : LAST, y = (tc / (R / 2)) % R + 1, z = tc / (R / 2 * R) + 1, x = 2 * (tc % (R / 2)) + 1;
+  // an x pair, four threads to the 2x2x2 cells that a thread of mg_patch has (see MgSums)
+  const int tc = active ? t : LAST, tb = tc >> 2, cb = tb % M::LP;
+  const int x = 2 * (cb % M::MX) + 1, y = 2 * (cb / M::MX) + 1 + (tc & 1), z = 2 * (tb / M::LP) + 1 + (tc >> 1 & 1);
   const int x1 = (y + z) & 1;   // which of x, x + 1 has colour 1
   const int id[2] = {nat(N, x + 1 - x1, y, z), nat(N, x + x1, y, z)};   // by colour
   T rh[2], gu[2] = {T(0), T(0)};
@@ -805,7 +823,7 @@ __device__ void mg_patch_cells(T* __restrict__ lds, const T* __restrict__ rho, c
       den += fabs(sol[id[c]]);
     }
     if (!active) num = den = T(0);
-    block_sum2<THREADS>(num, den, red);
+    block_sum2<THREADS / 16>(num, den, red);
     fell_back = !(num <= P.guess_tol * den);
     if (fell_back && active) sol[id[0]] = sol[id[1]] = T(0);
     __syncthreads();
@@ -861,7 +879,7 @@ __device__ void mg_patch_cells(T* __restrict__ lds, const T* __restrict__ rho, c
       ss += fabs(sol[id[c]]);
     }
     if (!active) sd = ss = T(0);
-    block_sum2<THREADS>(sd, ss, red);
+    block_sum2<THREADS / 16>(sd, ss, red);
     error = P.dh * P.dh * sd / ss;
     iter++;
   }

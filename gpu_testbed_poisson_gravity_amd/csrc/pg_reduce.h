@@ -41,6 +41,15 @@ __device__ __forceinline__ T wave_sum_dpp(T v) {
   return (lane_value(v, 0) + lane_value(v, 16)) + (lane_value(v, 32) + lane_value(v, 48));
 }
 
+// Sum of v[0..N-1] as a tree over adjacent halves.
+template <int N, typename T>
+__device__ __forceinline__ T tree_sum(const T* v) {
+  if constexpr (N == 1)
+    return v[0];
+  else
+    return tree_sum<N / 2>(v) + tree_sum<N - N / 2>(v + N / 2);
+}
+
 // Butterfly sum over the wavefront (partners 32, 16, ... 1 apart); with lanes beyond a shorter segment at zero, the bits
 // of the butterfly over that segment.
 __device__ __forceinline__ float wave_sum_butterfly(float v) {

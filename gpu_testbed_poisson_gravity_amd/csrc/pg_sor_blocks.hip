@@ -314,13 +314,6 @@ __device__ __forceinline__ void blocks_interpolate_odd(Block<GS, T, PLANES>& o, 
 }
 
 // Sum of the waves' values (one wave: each lane has it).
-template <int N, typename T>
-__device__ __forceinline__ T blocks_total(const T* red) {
-  if constexpr (N == 1)
-    return red[0];
-  else
-    return blocks_total<N / 2>(red) + blocks_total<N - N / 2>(red + N / 2);
-}
 template <int WAVES, typename T>
 __device__ __forceinline__ void blocks_put(T wave, T* red) {
   if (WAVES > 1 && (threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = wave;
@@ -330,7 +323,7 @@ __device__ __forceinline__ T blocks_get(T wave, const T* red) {
   if constexpr (WAVES == 1)
     return wave;
   else
-    return blocks_total<WAVES>(red);
+    return tree_sum<WAVES>(red);
 }
 
 // Sums of a and b over the workgroup, the same bits in every thread.  No barrier afterwards: the next use of the same
