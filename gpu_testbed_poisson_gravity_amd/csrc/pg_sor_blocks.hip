@@ -54,6 +54,12 @@ struct BlockGeo {
   static constexpr bool F64 = sizeof(T) == 8;
   static constexpr int HP = N / 2 + (GS == 1 || GS == 4 || (GS == 5 && !F64) ? 1 : 0);
   static constexpr int PL = N * HP + (GS == 1 && !F64 ? 12 : GS == 2 ? (F64 ? 3 : 1) : GS == 4 && F64 ? 2 : 0);
+  // One order of the stopping sums for both plane counts of FP64 ghost size 3, which the batch size chooses between: with two
+  // planes per thread, consecutive threads have the two halves of a four-plane chunk; with four, a thread adds its halves
+  // apart.  The sums over the threads are binary trees, so the rest of the order is the same.
+  static constexpr bool ONE_ORDER = F64 && GS == 3;
+  static constexpr int PARTS = ONE_ORDER && PLANES == 4 ? 2 : 1;   // sums per thread
+  __device__ static constexpr int part(int zi) { return PARTS == 2 ? zi >> 1 : 0; }
   // Pairs: a column's interior cells of one colour lie together, so that a thread's two are one 16-byte word; x pairs of
   // columns are XP words apart (their two Dirichlet cells last), rows RP.  A 16-byte read serves lanes 0-3, 12-15 and 20-27 of
   // 32 in a cycle, then the others; a write 8 lanes of 32 banks: XP is 2 modulo 16 and RP 8 modulo 16, without conflicts.
@@ -96,8 +102,11 @@ struct Block {
   __device__ __forceinline__ void init(int t) {
     active = t < G::OWNERS;
     if (!active) t = 0;   // reads stay in range; nothing is written
-    chunk = t / G::LP;
-    const int cb = t - chunk * G::LP, a = cb / G::MX, b = cb - a * G::MX;
+    const bool halves = G::ONE_ORDER && H == 2;
+    const int u = halves ? t >> 1 : t;
+    chunk = u / G::LP;
+    const int cb = u - chunk * G::LP, a = cb / G::MX, b = cb - a * G::MX;
+    if (halves) chunk = 2 * chunk + (t & 1);
     const int m = G::XMAJOR ? a : b, yb = G::XMAJOR ? b : a;
     x0 = 2 * m + 1;
     y0 = 2 * yb + 1;
@@ -489,11 +498,11 @@ __device__ __forceinline__ void blocks_patch(T* __restrict__ lds, const T* __res
   T res[2 * H], black[2 * H];   // residuals of one colour: the pass being tested, and the last second pass
   bool fell_back = false;
   if (P.init_mode >= 2 && P.guess_tol > T(0)) {
-    T num = T(0), den = T(0);
-    o.template each<1>(lds, [&](int q, int, int, int, T r) { num += fabs(res[q] = r); });
-    o.template each<0>(lds, [&](int q, int, int, int, T r) { num += fabs(black[q] = r); });
-    o.cells([&](int yy, int xx, int zi) { den += fabs(o.phi[yy][xx][zi]); });
-    if (!o.active) num = den = T(0);
+    T nums[G::PARTS] = {}, dens[G::PARTS] = {};
+    o.template each<1>(lds, [&](int q, int, int, int zi, T r) { nums[G::part(zi)] += fabs(res[q] = r); });
+    o.template each<0>(lds, [&](int q, int, int, int zi, T r) { nums[G::part(zi)] += fabs(black[q] = r); });
+    o.cells([&](int yy, int xx, int zi) { dens[G::part(zi)] += fabs(o.phi[yy][xx][zi]); });
+    T num = o.active ? tree_sum<G::PARTS>(nums) : T(0), den = o.active ? tree_sum<G::PARTS>(dens) : T(0);
     blocks_sum2<G::WAVES>(num, den, red);
     bool keep = num <= P.guess_tol * den;
     if constexpr (ORDERED) {
@@ -518,19 +527,20 @@ __device__ __forceinline__ void blocks_patch(T* __restrict__ lds, const T* __res
   const bool stall = P.term_mode == 0, relres = P.term_mode == 1;
   const int first_check = P.min_iter > 1 ? P.min_iter : 1;
   int it_done = P.max_iter, st = kStatusMaxIter;
-  T old = T(FLT_MAX), black_sum = T(0);   // Residual_Total_Old = __FLT_MAX__ (CPU_PoissonSolver_SOR.cpp:215)
+  T old = T(FLT_MAX), black_sum[G::PARTS] = {};   // Residual_Total_Old = __FLT_MAX__ (CPU_PoissonSolver_SOR.cpp:215)
   T prev1[2 * H], prev0[2 * H];           // residuals of the last iteration (stall rule, FP32)
 #pragma unroll
   for (int q = 0; q < 2 * H; q++) black[q] = prev1[q] = prev0[q] = T(0);
   for (int it = 0; it < P.max_iter; it++) {
-    T sum = T(0);
+    T sum[G::PARTS] = {};
     if (relres && it >= first_check && (it - first_check) % P.check_every == 0) {
       // first-colour residuals before the pass, second-colour ones |1 - omega| times those of the last pass
-      T num = T(0), den = T(0);
-      o.template each<1>(lds, [&](int q, int, int, int, T r) { num += fabs(res[q] = r); });
-      o.cells([&](int yy, int xx, int zi) { den += fabs(o.phi[yy][xx][zi]); });
-      num = num + P.damp * black_sum;
-      if (!o.active) num = den = T(0);
+      T dens[G::PARTS] = {};
+      o.template each<1>(lds, [&](int q, int, int, int zi, T r) { sum[G::part(zi)] += fabs(res[q] = r); });
+      o.cells([&](int yy, int xx, int zi) { dens[G::part(zi)] += fabs(o.phi[yy][xx][zi]); });
+#pragma unroll
+      for (int h = 0; h < G::PARTS; h++) sum[h] = sum[h] + P.damp * black_sum[h];
+      T num = o.active ? tree_sum<G::PARTS>(sum) : T(0), den = o.active ? tree_sum<G::PARTS>(dens) : T(0);
       blocks_sum2<G::WAVES>(num, den, red);
       bool stop = num <= P.rel_tol * den;
       if constexpr (ORDERED) {
@@ -554,7 +564,7 @@ __device__ __forceinline__ void blocks_patch(T* __restrict__ lds, const T* __res
     } else if (stall) {
       o.template each<1>(lds, [&](int q, int yy, int xx, int zi, T r) {
         if (ORDERED) res[q] = r;
-        sum += fabs(r);
+        sum[G::part(zi)] += fabs(r);
         o.phi[yy][xx][zi] = o.phi[yy][xx][zi] + P.w6 * r;
       });
     } else {
@@ -563,10 +573,11 @@ __device__ __forceinline__ void blocks_patch(T* __restrict__ lds, const T* __res
     o.template publish<1>(lds);
     __syncthreads();
     if (stall || (it + 1 >= first_check && (it + 1 - first_check) % P.check_every == 0)) {
-      black_sum = T(0);
+#pragma unroll
+      for (int h = 0; h < G::PARTS; h++) black_sum[h] = T(0);
       o.template each<0>(lds, [&](int q, int yy, int xx, int zi, T r) {
         if (ORDERED) black[q] = r;
-        black_sum += fabs(r);
+        black_sum[G::part(zi)] += fabs(r);
         o.phi[yy][xx][zi] = o.phi[yy][xx][zi] + P.w6 * r;
       });
     } else {
@@ -574,7 +585,9 @@ __device__ __forceinline__ void blocks_patch(T* __restrict__ lds, const T* __res
     }
     o.template publish<0>(lds);
     if (stall) {
-      T tot = o.active ? sum + black_sum : T(0);
+#pragma unroll
+      for (int h = 0; h < G::PARTS; h++) sum[h] = sum[h] + black_sum[h];
+      T tot = o.active ? tree_sum<G::PARTS>(sum) : T(0);
       T* r2 = red + 2 * G::WAVES;
       tot = wave_sum_dpp(tot);
       blocks_put<G::WAVES>(tot, r2);

@@ -138,3 +138,69 @@ def test_mg_slices_and_mixed_modes_stop_alike():
             _agree(res, k)
         plan.close()
         small.close()
+
+
+def _bisect(changes, lo, hi, steps=56):
+    """Neighbouring doubles: the last on lo's side for which changes(x) (an array) is false, with changes(hi) true."""
+    lo, hi = np.array(lo, np.float64), np.array(hi, np.float64)
+    assert not changes(lo).any() and changes(hi).all()
+    for _ in range(steps):
+        mid = lo + (hi - lo) / 2
+        c = changes(mid)
+        lo, hi = np.where(c, lo, mid), np.where(c, mid, hi)
+    assert np.all(hi - lo <= 2 * np.spacing(lo))
+    return lo
+
+
+ULPS = np.arange(-24, 25)
+FP64_SIZES = (512, 513, 700)   # ghost size 3: two planes per thread up to 512 patches, then four
+
+
+@pytest.mark.parametrize("rule, tol", [(pg.TERM_RELRES, 2.0), (pg.TERM_RELRES, 1.0), (pg.TERM_RELRES, 0.5),
+                                       (pg.TERM_REFERENCE, 0.0)])
+def test_fp64_sor_stops_alike_in_every_batch(rule, tol):
+    """The relaxation factor, the one double-precision setting of the rules, is put where a patch's count changes: in the
+    first iterations, while the residuals are far above round-off, so that a step of one unit in the last place moves the
+    sums by as little."""
+    gs, k = 3, 6
+    rho, cpot, _, _ = I.plummer(k, gs, seed=70, dtype=np.float64)
+    if rule == pg.TERM_RELRES:   # 2 to 4 iterations at a factor of 1, more below
+        opts, args, ends = dict(term_mode=rule, rel_tol=tol, init_mode=pg.INIT_ZERO), dict(sor_min_iter=0, sor_max_iter=20), (0.6, 1.0)
+    else:                        # the residual grows after two or three iterations above a factor of about 1.9
+        opts, args, ends = dict(term_mode=rule), dict(sor_min_iter=0, sor_max_iter=20), (1.6, 1.9)
+    few = _Solver(gs, np.float64, rho, cpot, k, **opts)
+    runs = [few] + [_Solver(gs, np.float64, rho, cpot, n, **opts) for n in FP64_SIZES]
+    most = few(sor_omega=ends[1], **args)[1]
+    for p in range(k):
+        at = _bisect(lambda w: few(sor_omega=float(w), **args)[1][p] <= most[p], *ends)
+        print(f"[case] f64 gs=3 rule {rule}: patch {p}, factors around {float(at):.6f}", flush=True)
+        got = {int(_agree([r(sor_omega=float(at + u * np.spacing(at)), **args) for r in runs], k)[1][p]) for u in ULPS}
+        assert len(got) > 1
+
+
+def test_fp64_sor_checks_guesses_alike_in_every_batch():
+    """The solution of a density as the guess, and the density scaled to where the guess fails (its tolerance is in single
+    precision)."""
+    gs, k, N = 3, 8, 14
+    rho, cpot, _, _ = I.plummer(k, gs, seed=70, dtype=np.float64)
+    cube = _Solver(gs, np.float64, rho, cpot, k, term_mode=pg.TERM_RELRES, gra_ghost_size=gs)(
+        sor_min_iter=10, sor_max_iter=400, sor_omega=1.6)[0]
+    assert cube.shape == (k, N, N, N)
+    guess = np.ascontiguousarray(cube[:, 1:-1, 1:-1, 1:-1])
+    ratio = np.abs(POI * rho).sum(axis=(1, 2, 3)) / np.abs(guess).sum(axis=(1, 2, 3))
+    opts = dict(term_mode=pg.TERM_RELRES, init_mode=pg.INIT_GUESS, guess_fallback_tol=float(ratio.max()))
+    args = dict(sor_min_iter=0, sor_max_iter=0)
+    few = _Solver(gs, np.float64, rho, cpot, k, guess=guess, **opts)
+
+    def fails(s):
+        few.rho.copy_(few.torch.as_tensor(rho * s[:, None, None, None]))
+        return (few(**args)[2] & pg.STATUS_FALLBACK) != 0
+
+    at = _bisect(fails, np.ones(k), np.full(k, 2 + ratio.max() / ratio.min()))
+    s = (at[:, None] + ULPS * np.spacing(at)[:, None]).reshape(-1)
+    pick = np.repeat(np.arange(k), ULPS.size)
+    many = rho[pick] * s[:, None, None, None], cpot[pick]
+    print(f"[case] f64 gs=3 guess check: {s.size} scales", flush=True)
+    res = [_Solver(gs, np.float64, *many, n, guess=guess[pick], **opts)(**args) for n in (s.size,) + FP64_SIZES]
+    fell = (_agree(res, s.size)[2] & pg.STATUS_FALLBACK).reshape(k, -1) != 0
+    assert np.all(fell.any(axis=1) & ~fell.all(axis=1))
