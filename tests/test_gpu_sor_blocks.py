@@ -138,3 +138,43 @@ def test_blocks_match_at_plane_changes(gs, n):
     """Batch sizes where the planes per thread change."""
     _same(gs, n, dict(term_mode=pg.TERM_REFERENCE), pg.solver_args(sor_min_iter=10, sor_max_iter=60, sor_omega=1.65,
                                                                    poi_coeff=POI, dt=0.5))
+
+
+@pytest.mark.parametrize("gs", [1, 3, 5])
+@pytest.mark.parametrize("what", ["zero", "nan"])
+def test_blocks_are_no_slower_on_patches_that_never_stop(gs, what):
+    """A patch of zeros, or with a NaN, ties at every comparison of the stall rule: the form that is chosen because it is
+    faster must not spend longer than the other one on sums whose order cannot matter."""
+    import torch
+
+    n = 256
+    rho, cpot, _ = _patches(gs, special=False)
+    at = np.arange(n) % K
+    rho, cpot = rho[at], cpot[at]
+    if what == "zero":
+        rho[0], cpot[0] = 0.0, 0.0
+    else:
+        rho[0, 1, 2, 3] = np.nan
+    rho, cpot = torch.as_tensor(rho).cuda(), torch.as_tensor(cpot).cuda()
+    args = pg.solver_args(sor_min_iter=10, sor_max_iter=1000, sor_omega=1.65, poi_coeff=POI, graacc=False)
+    ms, res = [], []
+    for fixed in (True, False):
+        with pg.Context(0) as ctx:
+            ctx.set_options(pot_ghost_size=gs, term_mode=pg.TERM_REFERENCE, fuse_gravity=0)
+            if fixed:
+                ctx.set_layout(gs, *DEFAULT[gs])
+            out, it = torch.zeros((n, 10, 10, 10), device="cuda"), torch.zeros(n, dtype=torch.int32, device="cuda")
+            best = 1e9
+            for _ in range(5):
+                e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+                e[0].record()
+                ctx.solve_device(rho, cpot, out, None, n, args, iters=it, stream=torch.cuda.current_stream().cuda_stream)
+                e[1].record()
+                torch.cuda.synchronize()
+                best = min(best, e[0].elapsed_time(e[1]))
+            ms.append(best)
+            res.append((out.cpu().numpy(), it.cpu().numpy()))
+    print(f"[case] one {what} patch of {n}, gs={gs}: one wavefront {ms[0]:.3f} ms, blocks {ms[1]:.3f} ms", flush=True)
+    assert res[0][1][0] == 1000 and np.array_equal(res[0][1], res[1][1])
+    assert np.array_equal(res[0][0][1:], res[1][0][1:])
+    assert ms[1] < ms[0]
