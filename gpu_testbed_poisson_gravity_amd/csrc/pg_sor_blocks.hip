@@ -407,8 +407,9 @@ struct OrderedSums {
 };
 
 // Whether the order of summation could decide between a and b: true where either is infinite (it may have overflowed in one
-// order only), false for NaN, which sums of absolute values have in every order or in none.
-__device__ __forceinline__ bool too_close(float a, float b) { return fabsf(a - b) <= 2e-5f * a + 2e-5f * b || a == b; }
+// order only), false for NaN, which sums of absolute values have in every order or in none.  FLT_MIN: products below it are
+// subnormal and round by more than the relative bound.
+__device__ __forceinline__ bool too_close(float a, float b) { return fabsf(a - b) <= 2e-5f * a + 2e-5f * b + FLT_MIN || a == b; }
 
 // Whether any thread's residuals differ from those of the last iteration.
 template <int WAVES, class B, int NQ>
@@ -614,7 +615,7 @@ __device__ __forceinline__ void blocks_patch(T* __restrict__ lds, const T* __res
       if (it + 1 >= P.min_iter) {
         bool grew = tot > old;
         if constexpr (ORDERED) {
-          if (too_close(tot, old) && (tot != old || blocks_moved<G::WAVES>(o, res, prev1, black, prev0, red))) {
+          if (__builtin_expect(too_close(tot, old), 0) && (tot != old || blocks_moved<G::WAVES>(o, res, prev1, black, prev0, red))) {
             float a = Ordered::column(o, res, lds);
             a += Ordered::column(o, black, lds);
             a = Ordered::wave(a, false, lds);

@@ -178,3 +178,34 @@ def test_blocks_are_no_slower_on_patches_that_never_stop(gs, what):
     assert res[0][1][0] == 1000 and np.array_equal(res[0][1], res[1][1])
     assert np.array_equal(res[0][0][1:], res[1][0][1:])
     assert ms[1] < ms[0]
+
+
+@pytest.mark.parametrize("gs", [1, 3, 5])
+def test_blocks_match_one_wavefront_among_subnormals(gs):
+    """Fields so small that the products in the stopping rules are subnormal and round by whole units."""
+    import torch
+
+    n, g = 256, pg.geometry(gs)
+    rng = np.random.default_rng(gs)
+    unit = np.float32(2.0 ** -149)   # the smallest subnormal
+    size = (rng.integers(1, 400, (n, 1, 1, 1))).astype(np.float32)
+    cpot = torch.as_tensor((rng.standard_normal((n,) + (g["C"],) * 3) * size).astype(np.float32).round() * unit).cuda()
+    rho = torch.as_tensor((rng.standard_normal((n,) + (g["R"],) * 3) * size).astype(np.float32).round() * unit / np.float32(POI)).cuda()
+    differ = 0
+    for tol in (0.9, 0.3, 0.1, 0.03):
+        for omega in (1.3, 1.7):
+            res = []
+            for fixed in (True, False):
+                with pg.Context(0) as ctx:
+                    ctx.set_options(pot_ghost_size=gs, term_mode=pg.TERM_RELRES, rel_tol=tol, fuse_gravity=0)
+                    if fixed:
+                        ctx.set_layout(gs, *DEFAULT[gs])
+                    out, it = torch.zeros((n, 10, 10, 10), device="cuda"), torch.zeros(n, dtype=torch.int32, device="cuda")
+                    args = pg.solver_args(sor_min_iter=0, sor_max_iter=40, sor_omega=omega, poi_coeff=POI, graacc=False)
+                    ctx.solve_device(rho, cpot, out, None, n, args, iters=it)
+                    torch.cuda.synchronize()
+                    res.append((out.cpu().numpy(), it.cpu().numpy()))
+            differ += (res[0][1] != res[1][1]).sum()
+            print(f"[case] subnormal gs={gs} tol={tol} omega={omega}: {np.unique(res[0][1]).size} counts, "
+                  f"{(res[0][1] != res[1][1]).sum()} differ", flush=True)
+    assert differ == 0
