@@ -124,6 +124,10 @@ struct pgamd_context {
   hipDeviceProp_t prop{};
   pgamd_options opt{};
   SorLayout layout{};
+  struct {
+    bool set = false;      // the caller has set a layout
+    int ppw = 0, pad = 0, blocks_to = 0;   // what the library used before that
+  } own[6];
   std::vector<hipStream_t> streams;
   int cap = 0;  // patches the device buffers hold
   float* d_rho = nullptr;
@@ -218,6 +222,7 @@ int pgamd_set_diagnose_device(int device_id, int* npatch_group, int* nstream, pg
   for (int g = 1; g <= 5; g++) {
     c->layout.ppw[g] = default_ppw(g);
     c->layout.pad[g] = default_pad(g);
+    c->layout.blocks_to[g] = sor_blocks_limit(g);
   }
   c->layout.ppw[0] = 1;
   c->layout.pad[0] = 0;
@@ -488,9 +493,24 @@ int pgamd_set_layout(pgamd_context* c, int gs, int ppw, int pad) {
   if (!supported_layout(gs, ppw, pad))
     return fail(PGAMD_ERR_ARG, "row padding %d is neither 0..3 nor the compact layout (ghost size 5, one patch "
                 "per wavefront)", pad);
-  c->layout.ppw[gs] = ppw;
-  c->layout.pad[gs] = pad;
-  c->layout.fixed[gs] = true;
+  SorLayout& lay = c->layout;
+  auto& own = c->own[gs];
+  if (own.set && ppw == own.ppw && pad == own.pad && (ppw != lay.ppw[gs] || pad != lay.pad[gs])) {
+    lay.ppw[gs] = ppw;   // put back
+    lay.pad[gs] = pad;
+    lay.blocks_to[gs] = own.blocks_to;
+    own.set = false;
+    return PGAMD_OK;
+  }
+  if (!own.set) {
+    own.ppw = lay.ppw[gs];
+    own.pad = lay.pad[gs];
+    own.blocks_to = lay.blocks_to[gs];
+    own.set = true;
+  }
+  lay.ppw[gs] = ppw;
+  lay.pad[gs] = pad;
+  lay.blocks_to[gs] = 0;
   return PGAMD_OK;
 }
 

@@ -137,7 +137,8 @@ struct ParamsByGs {
 // Per-ghost-size launch layout of the one-wavefront SOR kernel: patches per wavefront.  Chosen by the autotuner;
 // the default is the densest packing that fits one wavefront.
 struct SorLayout {
-  bool fixed[6];           // set by the caller: always the one-wavefront kernel, never the block form
+  int blocks_to[6];        // largest batch that runs in the block form instead, by gs (0: none; set by the caller, by the
+                           // autotuner, or sor_blocks_limit)
   int ppw[6];              // patches per wavefront, indexed by gs
   int pad[6];              // split-row padding in floats (bank-conflict avoidance), or kPadCompact, by gs
   int waves_per_cu;        // persistent kernel occupancy target
@@ -177,7 +178,7 @@ hipError_t launch_gravity64(const double* pot, double* flu, int npatch, int gra_
 // Block form of the SOR kernel, several wavefronts per patch.  FP32: same results and counts as the one-wavefront kernel;
 // wave_dpp is the order of its relative-residual sums (layouts with one patch per wavefront), ppw the patches per task of
 // a mixed batch.
-bool sor_blocks_better(int gs, int npatch);
+int sor_blocks_limit(int gs);
 hipError_t launch_sor_blocks(const UniformBatch& b, const SolveParams& p, bool wave_dpp, hipStream_t s);
 hipError_t launch_sor_blocks_tasks(const MixedBatch& b, const SolveParams& p, int gs, int ppw, int first, int count,
                                    hipStream_t s);

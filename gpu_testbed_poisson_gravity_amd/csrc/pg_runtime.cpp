@@ -125,7 +125,7 @@ int enqueue_mixed(pgamd_context* c, pgamd_plan* pl, const float* rho, const floa
     } else {
       const SorLayout& lay = ctx_layout(c);
       for (int g = kMaxGhost; g >= 1 && e == hipSuccess; g--)
-        e = !lay.fixed[g] && sor_blocks_better(g, pl->sor_count[g] * pl->sor_ppw[g])
+        e = pl->sor_count[g] * pl->sor_ppw[g] <= lay.blocks_to[g]
                 ? launch_sor_blocks_tasks(bs, P.p[g], g, pl->sor_ppw[g], pl->sor_first[g], pl->sor_count[g], st)
                 : launch_sor_tasks(bs, P.p[g], g, pl->sor_ppw[g], lay.pad[g], pl->sor_first[g], pl->sor_count[g], st);
     }

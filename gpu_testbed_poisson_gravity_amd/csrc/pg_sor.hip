@@ -1209,7 +1209,7 @@ int sor_uniform_blocks_per_cu(int gs, int ppw, int pad) {
 hipError_t launch_uniform(const UniformBatch& b, const SolveParams& p, const SorLayout& lay, hipStream_t s) {
   if (b.npatch <= 0) return hipSuccess;
   if (b.scheme == kSchemeMG) return launch_mg_uniform(b, p, s);
-  if (!lay.fixed[b.gs] && sor_blocks_better(b.gs, b.npatch)) return launch_sor_blocks(b, p, lay.ppw[b.gs] == 1, s);
+  if (b.npatch <= lay.blocks_to[b.gs]) return launch_sor_blocks(b, p, lay.ppw[b.gs] == 1, s);
   return launch_sor_uniform_dispatch(b, p, lay.ppw[b.gs], lay.pad[b.gs], s);
 }
 

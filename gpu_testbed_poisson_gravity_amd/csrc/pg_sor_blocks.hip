@@ -1,6 +1,6 @@
 // Red-black SOR with several wavefronts per patch on gfx950: every FP64 solve (the reference's FLOAT8 build, Makefile:22,
 // Header/Macro.h:35), and the FP32 batches for which it is faster than one wavefront per patch (pg_sor.hip): all at ghost
-// sizes 1 to 3, where that kernel leaves lanes idle, and those too small to fill the GPU with it (sor_blocks_better).
+// sizes 1 to 3, where that kernel leaves lanes idle, and those too small to fill the GPU with it (sor_blocks_limit).
 //
 // Reference behaviour reproduced (bit for bit at equal iteration counts):
 //   interpolation  CPU_PoissonSolver_SOR.cpp:110-203
@@ -35,6 +35,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cfloat>
+#include <climits>
 
 #include "pg_geometry.h"
 #include "pg_interp.h"
@@ -763,12 +764,12 @@ hipError_t launch_blocks(const UniformBatchT<typename PT::real>& b, const PT& p,
 
 }  // namespace
 
-// Where the block form is the faster one.  MI355X, us per call, one wavefront per patch (or group) / blocks, FP32 to 1e-5
+// Largest batch for which the block form is the faster one.  MI355X, us per call, one wavefront per patch (or group) / blocks, FP32 to 1e-5
 // from the interpolated start: GS 1, 8 patches 84 / 40, 4096: 109 / 69, 16384: 252 / 248; GS 2, 8: 83 / 39, 16384: 471 / 406
 // (25 of 32 lanes against 125 of 128); GS 3, 8: 87 / 43, 2048: 129 / 102, 16384: 821 / 633 (36 of 64 lanes against 108 of
 // 128); GS 4, 8: 95 / 43, 1024: 121 / 92, 1280: 124 / 124, 1536: 132 / 146; GS 5, 8: 103 / 44, 1024: 136 / 95, 1280:
 // 141 / 136, 1536: 148 / 150 (the one-wavefront kernel needs fewer reductions and reads once a launch fills the GPU).
-bool sor_blocks_better(int gs, int npatch) { return gs <= 3 || npatch <= 1024; }
+int sor_blocks_limit(int gs) { return gs <= 3 ? INT_MAX : 1024; }
 
 hipError_t launch_sor_blocks(const UniformBatch& b, const SolveParams& p, bool wave_dpp, hipStream_t s) {
   return launch_blocks(b, p, wave_dpp, s);

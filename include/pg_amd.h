@@ -186,8 +186,9 @@ int pgamd_scatter_patch_groups_device(int gra_ghost_size, int ngroup, const int*
  * is 5 runs that ghost size in the split layout with one float of padding).  Results do not depend on the
  * layout.  This is the autotuner's search space (pgamd_autotune); no reference counterpart: the reference
  * fixes its launch shapes per GPU generation with macros (Header/CUPOT.h:38-152).  Where several wavefronts per patch
- * are faster (ghost sizes 1..3, and up to 1024 patches at 4 and 5) the solve runs in that form, unless the caller has
- * set a layout for the ghost size with pgamd_set_layout; the results are the same. */
+ * are faster (ghost sizes 1..3, and up to 1024 patches at 4 and 5) the solve runs in that form instead; the results are the
+ * same.  pgamd_set_layout selects the one-wavefront kernel for its ghost size at every batch size, until the layout that the
+ * ghost size had before is put back (pgamd_get_layout before, pgamd_set_layout after). */
 #define PGAMD_LAYOUT_COMPACT 4
 int pgamd_set_layout(pgamd_context* ctx, int ghost_size, int patches_per_wave, int row_pad);
 int pgamd_get_layout(pgamd_context* ctx, int ghost_size, int* patches_per_wave, int* row_pad);
