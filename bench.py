@@ -235,7 +235,8 @@ def run_mixed(a):
         "dtype": "f32", "data": "synthetic",
         "config": {"workload": f"{n} patches, GS uniform in 1..5, densities {'/'.join(kinds)}, half SOR (omega by "
                                f"GS {OMEGA_BY_GS}) half MG (2+2 smoothing), rel. residual 1e-5, fused gravity, one "
-                               f"captured graph (one launch per ghost size and scheme), autotuned layouts {tuned}; start: "
+                               f"captured graph (one launch per ghost size and scheme), autotuned (one-wavefront layouts "
+                               f"{tuned}, several wavefronts per patch where faster); start: "
                                + ("learned warm start (guess check 1e-2)" if net is not None else "interpolation"),
                    "npatch": n},
         "network_ms": head["network_ms"], "solve_ms": sol, "sor": head["sor"], "mg": head["mg"],

@@ -496,10 +496,7 @@ int pgamd_set_layout(pgamd_context* c, int gs, int ppw, int pad) {
   SorLayout& lay = c->layout;
   auto& own = c->own[gs];
   if (own.set && ppw == own.ppw && pad == own.pad && (ppw != lay.ppw[gs] || pad != lay.pad[gs])) {
-    lay.ppw[gs] = ppw;   // put back
-    lay.pad[gs] = pad;
-    lay.blocks_to[gs] = own.blocks_to;
-    own.set = false;
+    ctx_set_layout(c, gs, ppw, pad, own.blocks_to);   // put back
     return PGAMD_OK;
   }
   if (!own.set) {
@@ -610,7 +607,16 @@ int pgamd_solve_device_f64(pgamd_context* c, const double* d_rho, const double* 
 namespace pgamd {
 
 const pgamd_options& ctx_options(const pgamd_context* c) { return c->opt; }
-SorLayout& ctx_layout(pgamd_context* c) { return c->layout; }
+const SorLayout& ctx_layout(const pgamd_context* c) { return c->layout; }
+void ctx_set_layout(pgamd_context* c, int gs, int ppw, int pad, int blocks_to) {
+  c->layout.ppw[gs] = ppw;
+  c->layout.pad[gs] = pad;
+  c->layout.blocks_to[gs] = blocks_to;
+  c->own[gs].set = false;
+}
+int ctx_own_blocks_limit(const pgamd_context* c, int gs) {
+  return c->own[gs].set ? c->own[gs].blocks_to : c->layout.blocks_to[gs];
+}
 int ctx_cu_count(const pgamd_context* c) { return c->prop.multiProcessorCount; }
 int ctx_device(const pgamd_context* c) { return c->device; }
 hipStream_t ctx_stream(const pgamd_context* c) { return c->streams[0]; }

@@ -16,7 +16,10 @@ int enqueue_solve(pgamd_context* c, const float* rho, const float* cpot, const f
                   float* flu, int npatch, const pgamd_solver_args& a, const SolveParams& p, int* iters, int* status,
                   hipStream_t st);
 const pgamd_options& ctx_options(const pgamd_context* c);
-SorLayout& ctx_layout(pgamd_context* c);
+const SorLayout& ctx_layout(const pgamd_context* c);
+// What the library chooses by itself from now on, in place of a layout that the caller had set.
+void ctx_set_layout(pgamd_context* c, int gs, int ppw, int pad, int blocks_to);
+int ctx_own_blocks_limit(const pgamd_context* c, int gs);   // SorLayout::blocks_to, or what it was before the caller set a layout
 int ctx_cu_count(const pgamd_context* c);
 int ctx_device(const pgamd_context* c);
 hipStream_t ctx_stream(const pgamd_context* c);

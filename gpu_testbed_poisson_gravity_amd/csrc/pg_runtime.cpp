@@ -390,10 +390,13 @@ int pgamd_graph_destroy(pgamd_graph* g) {
 
 // ---- autotuner ------------------------------------------------------------------------------------------
 //
-// Search space per ghost size: patches per wavefront in {1, 2, 4} (where they fit the 64 lanes) x row
-// padding in {0..3} floats, plus the compact layout at ghost size 5 (one patch per wavefront).  Each candidate runs one untimed solve and `repeats` timed ones on the caller's
-// stream-less default queue; the fastest mean wins.  The table is cached as a small JSON document:
-//   {"device": "<name>", "layouts": {"1": [ppw, pad], ..., "5": [ppw, pad]}}
+// Search space per ghost size: patches per wavefront in {1, 2, 4} (where they fit the 64 lanes) x row padding in {0..3}
+// floats, plus the compact layout at ghost size 5 (one patch per wavefront); and the form with several wavefronts per patch.
+// Each candidate runs one untimed solve and `repeats` timed ones on the context's first stream; the fastest mean wins.  The
+// block form is the one for small batches, so its result moves the largest batch that takes it: up to the timed size where it
+// won, to below that size where a layout did.  The table is cached as a small JSON document, the last part of which a file may
+// lack (the default limits then):
+//   {"device": "<name>", "layouts": {"1": [ppw, pad], ..., "5": [ppw, pad]}, "blocks_up_to": {"1": patches, ..., "5": patches}}
 
 #include <cstdio>
 #include <string>
@@ -422,38 +425,43 @@ int pgamd_autotune(pgamd_context* c, int gs, const float* rho, const float* cpot
   hipEvent_t e0, e1;
   if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess)
     return set_error(PGAMD_ERR_DEVICE, "hipEventCreate failed");
-  SorLayout& lay = ctx_layout(c);
+  const SorLayout& lay = ctx_layout(c);
   int bp = lay.ppw[gs], bd = lay.pad[gs];
   float bt = 1e30f;
   UniformBatch b{rho, cpot, nullptr, pot_out, nullptr, nullptr, nullptr, npatch, gs, PGAMD_SOR};
+  // mean time of a candidate; false if it does not launch on this device (e.g. LDS) or the device fails
+  auto timed = [&](auto launch, float& ms) {
+    if (launch() != hipSuccess) return false;
+    hipEventRecord(e0, st);
+    for (int r = 0; r < repeats; r++) launch();
+    hipEventRecord(e1, st);
+    if (hipEventSynchronize(e1) != hipSuccess) {
+      rc = set_error(PGAMD_ERR_DEVICE, "autotune synchronisation failed");
+      return false;
+    }
+    hipEventElapsedTime(&ms, e0, e1);
+    ms /= repeats;
+    return true;
+  };
+  float ms = 0.0f;
   for (int ppw : {1, 2, 4}) {
     if (!supported_ppw(gs, ppw)) continue;
-    for (int pad = 0; pad <= kPadCompact; pad++) {
+    for (int pad = 0; pad <= kPadCompact && rc == PGAMD_OK; pad++) {
       if (!supported_layout(gs, ppw, pad)) continue;
-      hipError_t e = launch_sor_uniform_dispatch(b, p, ppw, pad, st);
-      if (e != hipSuccess) continue;  // layout does not launch on this device (e.g. LDS): skip it
-      hipEventRecord(e0, st);
-      for (int r = 0; r < repeats; r++) launch_sor_uniform_dispatch(b, p, ppw, pad, st);
-      hipEventRecord(e1, st);
-      if (hipEventSynchronize(e1) != hipSuccess) {
-        hipEventDestroy(e0);
-        hipEventDestroy(e1);
-        return set_error(PGAMD_ERR_DEVICE, "autotune synchronisation failed");
-      }
-      float ms = 0.0f;
-      hipEventElapsedTime(&ms, e0, e1);
-      ms /= repeats;
-      if (ms < bt) {
+      if (timed([&] { return launch_sor_uniform_dispatch(b, p, ppw, pad, st); }, ms) && ms < bt) {
         bt = ms;
         bp = ppw;
         bd = pad;
       }
     }
   }
+  const bool blocks = rc == PGAMD_OK && timed([&] { return launch_sor_blocks(b, p, bp == 1, st); }, ms) && ms < bt;
   hipEventDestroy(e0);
   hipEventDestroy(e1);
-  lay.ppw[gs] = bp;
-  lay.pad[gs] = bd;
+  if (rc != PGAMD_OK) return rc;
+  if (blocks) bt = ms;
+  const int limit = ctx_own_blocks_limit(c, gs);
+  ctx_set_layout(c, gs, bp, bd, blocks ? std::max(limit, npatch) : std::min(limit, npatch - 1));
   if (best_ppw) *best_ppw = bp;
   if (best_pad) *best_pad = bd;
   if (best_ms) *best_ms = bt;
@@ -471,6 +479,8 @@ int pgamd_autotune_save(pgamd_context* c, const char* path) {
   dev = dev.substr(0, dev.find(';'));
   fprintf(f, "{\"device\": \"%s\", \"layouts\": {", dev.c_str());
   for (int g = 1; g <= kMaxGhost; g++) fprintf(f, "%s\"%d\": [%d, %d]", g > 1 ? ", " : "", g, lay.ppw[g], lay.pad[g]);
+  fprintf(f, "}, \"blocks_up_to\": {");
+  for (int g = 1; g <= kMaxGhost; g++) fprintf(f, "%s\"%d\": %d", g > 1 ? ", " : "", g, lay.blocks_to[g]);
   fprintf(f, "}}\n");
   fclose(f);
   return PGAMD_OK;
@@ -491,19 +501,22 @@ int pgamd_autotune_load(pgamd_context* c, const char* path) {
   dev = dev.substr(0, dev.find(';'));
   if (s.find("\"device\": \"" + dev + "\"") == std::string::npos)
     return set_error(PGAMD_ERR_STATE, "autotune cache was written for another device");
-  int ppw[6], pad[6];
+  int ppw[6], pad[6], blocks_to[6];
+  const size_t limits = s.find("\"blocks_up_to\": {");
   for (int g = 1; g <= kMaxGhost; g++) {
     const std::string key = "\"" + std::to_string(g) + "\": [";
     const size_t k = s.find(key);
     if (k == std::string::npos || sscanf(s.c_str() + k + key.size(), "%d, %d", &ppw[g], &pad[g]) != 2 ||
         !supported_layout(g, ppw[g], pad[g]))
       return set_error(PGAMD_ERR_ARG, "malformed autotune cache");
+    blocks_to[g] = sor_blocks_limit(g);
+    if (limits == std::string::npos) continue;
+    const std::string entry = "\"" + std::to_string(g) + "\": ";
+    const size_t b = s.find(entry, limits);
+    if (b == std::string::npos || sscanf(s.c_str() + b + entry.size(), "%d", &blocks_to[g]) != 1 || blocks_to[g] < 0)
+      return set_error(PGAMD_ERR_ARG, "malformed autotune cache");
   }
-  SorLayout& lay = ctx_layout(c);
-  for (int g = 1; g <= kMaxGhost; g++) {
-    lay.ppw[g] = ppw[g];
-    lay.pad[g] = pad[g];
-  }
+  for (int g = 1; g <= kMaxGhost; g++) ctx_set_layout(c, g, ppw[g], pad[g], blocks_to[g]);
   return PGAMD_OK;
 }
 

@@ -186,13 +186,14 @@ int pgamd_scatter_patch_groups_device(int gra_ghost_size, int ngroup, const int*
  * is 5 runs that ghost size in the split layout with one float of padding).  Results do not depend on the
  * layout.  This is the autotuner's search space (pgamd_autotune); no reference counterpart: the reference
  * fixes its launch shapes per GPU generation with macros (Header/CUPOT.h:38-152).  Where several wavefronts per patch
- * are faster (ghost sizes 1..3, and up to 1024 patches at 4 and 5) the solve runs in that form instead; the results are the
- * same.  pgamd_set_layout selects the one-wavefront kernel for its ghost size at every batch size, until the layout that the
- * ghost size had before is put back (pgamd_get_layout before, pgamd_set_layout after). */
+ * are faster (ghost sizes 1..3, and up to 1024 patches at 4 and 5, unless pgamd_autotune has found another limit) the solve
+ * runs in that form instead; the results are the same.  pgamd_set_layout selects the one-wavefront kernel for its ghost size
+ * at every batch size, until the layout that the ghost size had before is put back (pgamd_get_layout before, pgamd_set_layout
+ * after), or pgamd_autotune or pgamd_autotune_load chooses again. */
 #define PGAMD_LAYOUT_COMPACT 4
 int pgamd_set_layout(pgamd_context* ctx, int ghost_size, int patches_per_wave, int row_pad);
 int pgamd_get_layout(pgamd_context* ctx, int ghost_size, int* patches_per_wave, int* row_pad);
-/* Residency of the SOR kernel at the context's layout for one ghost size: workgroups (one wavefront each) the
+/* Residency of the one-wavefront SOR kernel at the context's layout for one ghost size: workgroups (one wavefront each) the
  * device keeps resident per CU, and the patches that makes (times patches per wavefront), from the kernel's
  * registers and LDS (hipOccupancyMaxActiveBlocksPerMultiprocessor).  No reference counterpart. */
 int pgamd_layout_occupancy(pgamd_context* ctx, int ghost_size, int* workgroups_per_cu, int* patches_per_cu);
@@ -239,10 +240,12 @@ int pgamd_solve_device_f64(pgamd_context* ctx, const double* d_rho, const double
                            double* d_pot_out, double* d_flu, int npatch, const pgamd_solver_args_f64* args,
                            int* d_iters, int* d_status, void* stream);
 
-/* Autotuner: times every supported layout of one ghost size on the caller's device batch (SOR with the
- * context's options, gravity off; repeats >= 1 timed solves per candidate after one warm-up), keeps the
- * fastest in the context and returns it.  d_pot_out is overwritten.  The layout table can be saved and
- * reloaded as JSON, keyed by device name. */
+/* Autotuner: times every supported layout of one ghost size, and the form with several wavefronts per patch, on the
+ * caller's device batch (SOR with the context's options, gravity off; repeats >= 1 timed solves per candidate after one
+ * warm-up) and keeps the fastest in the context, also over a layout set before.  best_ppw and best_pad are the fastest layout,
+ * best_ms the time of what the context now runs for such a batch: that layout, or the other form, which is then taken up to at
+ * least this batch size (where the layout wins, only below it).  d_pot_out is overwritten.  The table of layouts and limits
+ * can be saved and reloaded as JSON, keyed by device name. */
 int pgamd_autotune(pgamd_context* ctx, int ghost_size, const float* d_rho, const float* d_pot_in, float* d_pot_out,
                    int npatch, const pgamd_solver_args* args, int repeats, int* best_ppw, int* best_pad,
                    float* best_ms);
