@@ -175,6 +175,14 @@ int ensure_streams(pgamd_context* c, int n) {
   return PGAMD_OK;
 }
 
+// Whether copies from and to the array p run without holding the host.
+bool pinned(const void* p) {
+  hipPointerAttribute_t at{};
+  if (hipPointerGetAttributes(&at, p) == hipSuccess) return at.type != hipMemoryTypeUnregistered;
+  (void)hipGetLastError();   // an address the runtime does not know
+  return false;
+}
+
 int ensure_slices(pgamd_context* c) {
   for (auto& s : c->copy)
     if (!s) HIP_TRY(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
@@ -418,16 +426,26 @@ int pgamd_asyn_poisson_gravity_solver(pgamd_context* c, const float* h_rho, floa
   // hardware queue with the solves (3.74 ms), and copying out by a kernel of 16 workgroups gains 1%.
   // Host arrays that share memory (other than the fluid with itself) keep the sequence: an early slice's results would
   // overwrite what a later one reads.
+  // Copies of pageable arrays hold the host, so only the solve hides behind them: two slices, and the sequence for gravity
+  // alone.  Sequence / as many slices as with pinned arrays / this rule, pageable: 8192 GS-1 patches, Poisson only, 3.04 /
+  // 3.15 / 3.07 ms; 2048 GS-5 patches 4.27 / 4.23 / 4.11; gravity alone, 1024: 1.04 / 1.13 / 1.04, 8192: 8.65 / 8.90 / 8.65.
+  // Gravity alone from pinned arrays has only its copies to overlap: 1024 patches 481 us in sequence, 490 in slices, 1536 702
+  // and 664.
   auto apart = [&](const float* x, size_t xn, const float* y, size_t yn) {
     const uintptr_t a0 = (uintptr_t)x, b0 = (uintptr_t)y;
     return !x || !y || a0 + 4 * npatch * xn <= b0 || b0 + 4 * npatch * yn <= a0;
   };
-  if (gpu_nstream == 1 && npatch >= 2 * kSlicePatches && apart(h_pot_out, c->out_n, h_rho, c->rho_n) &&
+  int max_slices = 1;
+  if (gpu_nstream == 1 && npatch >= (poisson ? 2 : 3) * kSlicePatches) {
+    const bool free_host = (!poisson || (pinned(h_rho) && pinned(h_pot_in))) && pinned(h_pot_out) && (!graacc || pinned(h_flu));
+    max_slices = free_host ? kMaxSlices : poisson ? 2 : 1;
+  }
+  if (max_slices > 1 && apart(h_pot_out, c->out_n, h_rho, c->rho_n) &&
       apart(h_pot_out, c->out_n, h_pot_in, c->cpot_n) && apart(h_pot_out, c->out_n, h_flu, flu_n) &&
       apart(h_flu, flu_n, h_rho, c->rho_n) && apart(h_flu, flu_n, h_pot_in, c->cpot_n)) {
     size_t at[kMaxSlices + 1] = {};
     int ns = 0;
-    while (ns + 1 < kMaxSlices && npatch - at[ns] >= 2 * kSlicePatches) {
+    while (ns + 1 < max_slices && npatch - at[ns] >= 2 * kSlicePatches) {
       at[ns + 1] = at[ns] + (npatch - at[ns]) / 2 / 64 * 64;
       ns++;
     }

@@ -70,3 +70,11 @@ def test_overlapping_arrays_keep_the_sequence():
             res.append((both[:h_out.size].copy(), h_flu.copy()))
     for x, y in zip(*res):
         assert np.array_equal(x, y)
+
+
+@pytest.mark.parametrize("pinned", [True, False])
+@pytest.mark.parametrize("gs, n, poisson", [(1, 1528, False), (2, 1544, False), (2, 2056, True), (4, 4104, True)])
+def test_slices_match_at_their_limits(gs, n, poisson, pinned):
+    """Gravity alone around its smallest sliced batch, and batches of several slices that pageable arrays get two of; the
+    test's second call of each is 8 patches smaller."""
+    test_slices_match_the_sequence(gs, pg.SOR, n, poisson, True, pinned)
