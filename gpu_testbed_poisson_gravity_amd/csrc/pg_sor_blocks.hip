@@ -47,7 +47,8 @@
 namespace pgamd {
 namespace {
 
-template <int GS, typename T, int PLANES>
+// HELP: workgroup of HELP times the waves that own cells; the others only share the work before and after the iterations.
+template <int GS, typename T, int PLANES, int HELP = 1>
 struct BlockGeo {
   static constexpr Geo g = geo_of(GS);
   static constexpr int N = g.N, R = g.R, C = g.C, U = g.U;
@@ -55,7 +56,10 @@ struct BlockGeo {
   static constexpr int H = PLANES;                        // planes per thread
   static constexpr int CHUNKS = R / H;
   static constexpr int OWNERS = LP * CHUNKS;
-  static constexpr int THREADS = (OWNERS + 63) / 64 * 64;
+  static constexpr int THREADS = (OWNERS + 63) / 64 * 64 * HELP;
+  static constexpr int FACES = HELP > 1 ? OWNERS : 0;     // first thread with a face's coarse cell (interpolation)
+  static constexpr int EDGES = HELP > 1 ? FACES + 6 * LP : 0;
+  static_assert(HELP == 1 || (OWNERS == 64 && EDGES + 12 * MX + 8 <= THREADS), "one wave of owners, one item per helper");
   static constexpr bool F64 = sizeof(T) == 8;
   static constexpr int HP = N / 2 + (GS == 1 || GS == 4 || (GS == 5 && !F64) ? 1 : 0);
   static constexpr int PL = N * HP + (GS == 1 && !F64 ? 12 : GS == 2 ? (F64 ? 3 : 1) : GS == 4 && F64 ? 2 : 0);
@@ -74,7 +78,7 @@ struct BlockGeo {
   static constexpr bool XMAJOR = GS >= 3 && !PAIRS;       // lane order within a plane: x blocks slow
   static constexpr int CS = PAIRS ? N * RP : N * PL;      // words per colour
   static constexpr int NC = C - 2;                        // coarse cells with children in the cube, per axis
-  static constexpr int WAVES = THREADS / 64;
+  static constexpr int WAVES = THREADS / 64 / HELP;       // with cells
   static constexpr int RED = 2 * CS;                      // two pairs of wave sums
   static constexpr int SCRATCH = RED + 4 * WAVES;         // FP32: 2H values per column (ordered sums), one result
   static constexpr int WORDS = SCRATCH + (F64 ? 0 : 2 * H * 64 + 1);
@@ -92,9 +96,9 @@ struct BlockGeo {
 };
 
 // A thread's cells.
-template <int GS, typename T, int PLANES>
+template <int GS, typename T, int PLANES, int HELP = 1>
 struct Block {
-  using G = BlockGeo<GS, T, PLANES>;
+  using G = BlockGeo<GS, T, PLANES, HELP>;
   static constexpr int H = G::H;
   T phi[2][2][H], cr[2][2][H];   // [yy][xx][zi]; cr = Const*rho
   int x0, y0, z0;                // cube coordinates of the first cell, all odd
@@ -266,13 +270,15 @@ __device__ __forceinline__ void blocks_interpolate_even(T* __restrict__ lds, int
 // Odd ghost sizes: a thread's block is whole coarse cells, whose children go straight to its registers (interior: with
 // the interpolated start); the faces' coarse cells are shared out and their children written once the staged coarse
 // potential has been read.  The cube's edges and corners, which no stencil reads, go straight to a window that has them.
-template <int GS, typename T, int PLANES>
-__device__ __forceinline__ void blocks_interpolate_odd(Block<GS, T, PLANES>& o, T* __restrict__ lds, T* __restrict__ out, bool interior,
+template <int GS, typename T, int PLANES, int HELP>
+__device__ __forceinline__ void blocks_interpolate_odd(Block<GS, T, PLANES, HELP>& o, T* __restrict__ lds, T* __restrict__ out, bool interior,
                                                        bool whole, int int_scheme, int t) {
-  using G = BlockGeo<GS, T, PLANES>;
+  using G = BlockGeo<GS, T, PLANES, HELP>;
   constexpr int NC = G::NC, N = G::N, C = G::C, MX = G::MX, LP = G::LP, FI = (6 * LP + G::THREADS - 1) / G::THREADS;
+  // helpers take the faces and the edges while the owners are at their blocks
+  auto face_item = [&](int u) { return (unsigned)(t - G::FACES + u * G::THREADS); };
   static_assert(G::U == 1 && NC == MX + 2, "blocks are coarse cells");
-  if (interior) {
+  if (interior && (HELP == 1 || o.active)) {
 #pragma unroll
     for (int kk = 0; kk < G::H / 2; kk++) {
       T ch[2][2][2];
@@ -284,8 +290,8 @@ __device__ __forceinline__ void blocks_interpolate_odd(Block<GS, T, PLANES>& o, 
   T face[FI][4];
 #pragma unroll
   for (int u = 0; u < FI; u++) {
-    const int q = t + u * G::THREADS, f = q / LP, r = q - f * LP, b = r / MX, a = r - b * MX, ax = f >> 1, end = f & 1 ? NC : 1;
-    if (q < 6 * LP) {
+    const int q = face_item(u), f = q / LP, r = q - f * LP, b = r / MX, a = r - b * MX, ax = f >> 1, end = f & 1 ? NC : 1;
+    if ((unsigned)q < 6 * LP) {
       T ch[2][2][2];
       blocks_children<C>(lds, ax == 0 ? end : a + 2, ax == 0 ? a + 2 : ax == 1 ? end : b + 2, ax == 2 ? end : b + 2, int_scheme, ch);
       const int s = 1 - (f & 1);   // the child on the Dirichlet layer
@@ -299,7 +305,7 @@ __device__ __forceinline__ void blocks_interpolate_odd(Block<GS, T, PLANES>& o, 
     }
   }
   if (whole) {
-    for (int q = t; q < 12 * MX + 8; q += G::THREADS) {
+    for (int q = t >= G::EDGES ? t - G::EDGES : t + G::THREADS; q < 12 * MX + 8; q += G::THREADS) {
       const int ed = q / MX, ax = q < 12 * MX ? ed >> 2 : 3, bits = q < 12 * MX ? ed & 3 : q - 12 * MX, a = q - ed * MX + 2;
       const int e0 = bits & 1 ? NC : 1, e1 = bits & 2 ? NC : 1, e2 = bits & 4 ? NC : 1;
       const int i = ax == 0 ? a : e0, j = ax == 1 ? a : ax == 0 ? e0 : e1, k = ax == 2 ? a : ax == 3 ? e2 : e1;
@@ -316,8 +322,8 @@ __device__ __forceinline__ void blocks_interpolate_odd(Block<GS, T, PLANES>& o, 
   __syncthreads();
 #pragma unroll
   for (int u = 0; u < FI; u++) {
-    const int q = t + u * G::THREADS, f = q / LP, r = q - f * LP, b = r / MX, a = r - b * MX, d = f & 1 ? N - 1 : 0;
-    if (q < 6 * LP) {
+    const int q = face_item(u), f = q / LP, r = q - f * LP, b = r / MX, a = r - b * MX, d = f & 1 ? N - 1 : 0;
+    if ((unsigned)q < 6 * LP) {
 #pragma unroll
       for (int e = 0; e < 4; e++) {
         const int p = 2 * a + 1 + (e & 1), w = 2 * b + 1 + (e >> 1);
@@ -340,17 +346,30 @@ __device__ __forceinline__ T blocks_get(T wave, const T* red) {
     return tree_sum<WAVES>(red);
 }
 
+// Orders the LDS accesses of the threads with cells: a workgroup barrier, or beside helpers, where one wave has them all, only a
+// compiler fence (a wave's LDS operations execute in order).
+template <class G>
+__device__ __forceinline__ void blocks_sync() {
+  if (G::THREADS > 64 * G::WAVES) {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  } else {
+    __syncthreads();
+  }
+}
+
 // Sums of a and b over the workgroup, the same bits in every thread.  No barrier afterwards: the next use of the same
 // `red` comes after at least one other barrier.
-template <int WAVES, typename T>
+template <class G, typename T>
 __device__ __forceinline__ void blocks_sum2(T& a, T& b, T* red) {
   a = wave_sum_dpp(a);
   b = wave_sum_dpp(b);
-  blocks_put<WAVES>(a, red);
-  blocks_put<WAVES>(b, red + WAVES);
-  __syncthreads();
-  a = blocks_get<WAVES>(a, red);
-  b = blocks_get<WAVES>(b, red + WAVES);
+  blocks_put<G::WAVES>(a, red);
+  blocks_put<G::WAVES>(b, red + G::WAVES);
+  blocks_sync<G>();
+  a = blocks_get<G::WAVES>(a, red);
+  b = blocks_get<G::WAVES>(b, red + G::WAVES);
 }
 
 // The sums of the one-wavefront kernel (FP32): per column, the cells of a colour from the bottom up, lane `column` of the
@@ -462,17 +481,17 @@ __device__ __forceinline__ void blocks_gravity(const T* __restrict__ lds, Idx id
 }
 
 // One patch.  wave_dpp (FP32): the one-wavefront kernel's order of the relative-residual sums.
-template <int GS, int PLANES, typename PT, typename T = typename PT::real>
+template <int GS, int PLANES, int HELP, typename PT, typename T = typename PT::real>
 __device__ __forceinline__ void blocks_patch(T* __restrict__ lds, const T* __restrict__ rho, const T* __restrict__ cpot,
                                              const T* __restrict__ guess, T* __restrict__ out, T* __restrict__ flu,
                                              int* iters, int* status, const PT& P, bool wave_dpp) {
-  using G = BlockGeo<GS, T, PLANES>;
+  using G = BlockGeo<GS, T, PLANES, HELP>;
   using Ordered = OrderedSums<GS, PLANES>;
   constexpr int N = G::N, R = G::R, H = G::H, THREADS = G::THREADS;
   constexpr bool ORDERED = !G::F64;
   const int t = threadIdx.x;
   T* red = lds + G::RED;
-  Block<GS, T, PLANES> o;
+  Block<GS, T, PLANES, HELP> o;
   o.init(t);
 
   // Const*rho first where that pays: its loads run beside those of the coarse potential; after the interpolation they are a
@@ -514,137 +533,139 @@ __device__ __forceinline__ void blocks_patch(T* __restrict__ lds, const T* __res
   }
   __syncthreads();
 
-  // B'. a caller guess whose relative residual exceeds guess_tol is replaced by the zero guess
-  T res[2 * H], black[2 * H];   // residuals of one colour: the pass being tested, and the last second pass
   bool fell_back = false;
-  if (P.init_mode >= 2 && P.guess_tol > T(0)) {
-    T nums[G::PARTS] = {}, dens[G::PARTS] = {};
-    o.template each<1>(lds, [&](int q, int, int, int zi, T r) { nums[G::part(zi)] += fabs(res[q] = r); });
-    o.template each<0>(lds, [&](int q, int, int, int zi, T r) { nums[G::part(zi)] += fabs(black[q] = r); });
-    o.cells([&](int yy, int xx, int zi) { dens[G::part(zi)] += fabs(o.phi[yy][xx][zi]); });
-    T num = o.active ? tree_sum<G::PARTS>(nums) : T(0), den = o.active ? tree_sum<G::PARTS>(dens) : T(0);
-    blocks_sum2<G::WAVES>(num, den, red);
-    bool keep = num <= P.guess_tol * den;
-    if constexpr (ORDERED) {
-      if (too_close(num, P.guess_tol * den)) {
-        float n1 = Ordered::column(o, res, lds);
-        n1 += Ordered::column(o, black, lds);
-        n1 = Ordered::wave(n1, false, lds);
-        keep = n1 <= P.guess_tol * Ordered::wave(Ordered::column_phi(lds), false, lds);
-      }
-    }
-    fell_back = !keep;
-    __syncthreads();
-    if (fell_back) {
-      o.cells([&](int yy, int xx, int zi) { o.phi[yy][xx][zi] = T(0); });
-      o.template publish<0>(lds);
-      o.template publish<1>(lds);
-    }
-    __syncthreads();
-  }
-
-  // C. red-black iterations: pass 0 updates the cells with x + y + z odd (colour 1), pass 1 the others
-  const bool stall = P.term_mode == 0, relres = P.term_mode == 1;
-  const int first_check = P.min_iter > 1 ? P.min_iter : 1;
   int it_done = P.max_iter, st = kStatusMaxIter;
-  T old = T(FLT_MAX), black_sum[G::PARTS] = {};   // Residual_Total_Old = __FLT_MAX__ (CPU_PoissonSolver_SOR.cpp:215)
-  T prev1[2 * H], prev0[2 * H];           // residuals of the last iteration (stall rule, FP32)
-#pragma unroll
-  for (int q = 0; q < 2 * H; q++) black[q] = prev1[q] = prev0[q] = T(0);
-  for (int it = 0; it < P.max_iter; it++) {
-    T sum[G::PARTS] = {};
-    if (relres && it >= first_check && (it - first_check) % P.check_every == 0) {
-      // first-colour residuals before the pass, second-colour ones |1 - omega| times those of the last pass
-      T dens[G::PARTS] = {};
-      o.template each<1>(lds, [&](int q, int, int, int zi, T r) { sum[G::part(zi)] += fabs(res[q] = r); });
+  if (HELP == 1 || o.active) {   // helpers wait for the owners after the iterations
+    // B'. a caller guess whose relative residual exceeds guess_tol is replaced by the zero guess
+    T res[2 * H], black[2 * H];   // residuals of one colour: the pass being tested, and the last second pass
+    if (P.init_mode >= 2 && P.guess_tol > T(0)) {
+      T nums[G::PARTS] = {}, dens[G::PARTS] = {};
+      o.template each<1>(lds, [&](int q, int, int, int zi, T r) { nums[G::part(zi)] += fabs(res[q] = r); });
+      o.template each<0>(lds, [&](int q, int, int, int zi, T r) { nums[G::part(zi)] += fabs(black[q] = r); });
       o.cells([&](int yy, int xx, int zi) { dens[G::part(zi)] += fabs(o.phi[yy][xx][zi]); });
-#pragma unroll
-      for (int h = 0; h < G::PARTS; h++) sum[h] = sum[h] + P.damp * black_sum[h];
-      T num = o.active ? tree_sum<G::PARTS>(sum) : T(0), den = o.active ? tree_sum<G::PARTS>(dens) : T(0);
-      blocks_sum2<G::WAVES>(num, den, red);
-      bool stop = num <= P.rel_tol * den;
+      T num = o.active ? tree_sum<G::PARTS>(nums) : T(0), den = o.active ? tree_sum<G::PARTS>(dens) : T(0);
+      blocks_sum2<G>(num, den, red);
+      bool keep = num <= P.guess_tol * den;
       if constexpr (ORDERED) {
-        if (too_close(num, P.rel_tol * den)) {
+        if (too_close(num, P.guess_tol * den)) {
           float n1 = Ordered::column(o, res, lds);
-          n1 = n1 + P.damp * Ordered::column(o, black, lds);
-          n1 = Ordered::wave(n1, wave_dpp, lds);
-          stop = n1 <= P.rel_tol * Ordered::wave(Ordered::column_phi(lds), wave_dpp, lds);
+          n1 += Ordered::column(o, black, lds);
+          n1 = Ordered::wave(n1, false, lds);
+          keep = n1 <= P.guess_tol * Ordered::wave(Ordered::column_phi(lds), false, lds);
         }
       }
-      if (stop) {
-        it_done = it;
-        st = kStatusConverged;
-        break;
+      fell_back = !keep;
+      blocks_sync<G>();
+      if (fell_back) {
+        o.cells([&](int yy, int xx, int zi) { o.phi[yy][xx][zi] = T(0); });
+        o.template publish<0>(lds);
+        o.template publish<1>(lds);
       }
-#pragma unroll
-      for (int q = 0; q < 2 * H; q++) {
-        T& ph = o.phi[q & 1][o.xx_of(1, q & 1, q >> 1)][q >> 1];
-        ph = ph + P.w6 * res[q];
-      }
-    } else if (stall) {
-      o.template each<1>(lds, [&](int q, int yy, int xx, int zi, T r) {
-        if (ORDERED) res[q] = r;
-        sum[G::part(zi)] += fabs(r);
-        o.phi[yy][xx][zi] = o.phi[yy][xx][zi] + P.w6 * r;
-      });
-    } else {
-      o.template each<1>(lds, [&](int, int yy, int xx, int zi, T r) { o.phi[yy][xx][zi] = o.phi[yy][xx][zi] + P.w6 * r; });
+      blocks_sync<G>();
     }
-    o.template publish<1>(lds);
-    __syncthreads();
-    if (stall || (it + 1 >= first_check && (it + 1 - first_check) % P.check_every == 0)) {
+
+    // C. red-black iterations: pass 0 updates the cells with x + y + z odd (colour 1), pass 1 the others
+    const bool stall = P.term_mode == 0, relres = P.term_mode == 1;
+    const int first_check = P.min_iter > 1 ? P.min_iter : 1;
+    T old = T(FLT_MAX), black_sum[G::PARTS] = {};   // Residual_Total_Old = __FLT_MAX__ (CPU_PoissonSolver_SOR.cpp:215)
+    T prev1[2 * H], prev0[2 * H];           // residuals of the last iteration (stall rule, FP32)
 #pragma unroll
-      for (int h = 0; h < G::PARTS; h++) black_sum[h] = T(0);
-      o.template each<0>(lds, [&](int q, int yy, int xx, int zi, T r) {
-        if (ORDERED) black[q] = r;
-        black_sum[G::part(zi)] += fabs(r);
-        o.phi[yy][xx][zi] = o.phi[yy][xx][zi] + P.w6 * r;
-      });
-    } else {
-      o.template each<0>(lds, [&](int, int yy, int xx, int zi, T r) { o.phi[yy][xx][zi] = o.phi[yy][xx][zi] + P.w6 * r; });
-    }
-    o.template publish<0>(lds);
-    if (stall) {
+    for (int q = 0; q < 2 * H; q++) black[q] = prev1[q] = prev0[q] = T(0);
+    for (int it = 0; it < P.max_iter; it++) {
+      T sum[G::PARTS] = {};
+      if (relres && it >= first_check && (it - first_check) % P.check_every == 0) {
+        // first-colour residuals before the pass, second-colour ones |1 - omega| times those of the last pass
+        T dens[G::PARTS] = {};
+        o.template each<1>(lds, [&](int q, int, int, int zi, T r) { sum[G::part(zi)] += fabs(res[q] = r); });
+        o.cells([&](int yy, int xx, int zi) { dens[G::part(zi)] += fabs(o.phi[yy][xx][zi]); });
 #pragma unroll
-      for (int h = 0; h < G::PARTS; h++) sum[h] = sum[h] + black_sum[h];
-      T tot = o.active ? tree_sum<G::PARTS>(sum) : T(0);
-      T* r2 = red + 2 * G::WAVES;
-      tot = wave_sum_dpp(tot);
-      blocks_put<G::WAVES>(tot, r2);
-      __syncthreads();
-      tot = blocks_get<G::WAVES>(tot, r2);
-      if (it + 1 >= P.min_iter) {
-        bool grew = tot > old;
+        for (int h = 0; h < G::PARTS; h++) sum[h] = sum[h] + P.damp * black_sum[h];
+        T num = o.active ? tree_sum<G::PARTS>(sum) : T(0), den = o.active ? tree_sum<G::PARTS>(dens) : T(0);
+        blocks_sum2<G>(num, den, red);
+        bool stop = num <= P.rel_tol * den;
         if constexpr (ORDERED) {
-          if (__builtin_expect(too_close(tot, old), 0) && (tot != old || blocks_moved<G::WAVES>(o, res, prev1, black, prev0, red))) {
-            float a = Ordered::column(o, res, lds);
-            a += Ordered::column(o, black, lds);
-            a = Ordered::wave(a, false, lds);
-            float b = FLT_MAX;
-            if (it > 0) {
-              b = Ordered::column(o, prev1, lds);
-              b += Ordered::column(o, prev0, lds);
-              b = Ordered::wave(b, false, lds);
-            }
-            grew = a > b;
+          if (too_close(num, P.rel_tol * den)) {
+            float n1 = Ordered::column(o, res, lds);
+            n1 = n1 + P.damp * Ordered::column(o, black, lds);
+            n1 = Ordered::wave(n1, wave_dpp, lds);
+            stop = n1 <= P.rel_tol * Ordered::wave(Ordered::column_phi(lds), wave_dpp, lds);
           }
         }
-        if (grew) {
-          it_done = it + 1;
+        if (stop) {
+          it_done = it;
           st = kStatusConverged;
           break;
         }
-      }
-      old = tot;
-      if (ORDERED) {
 #pragma unroll
         for (int q = 0; q < 2 * H; q++) {
-          prev1[q] = res[q];
-          prev0[q] = black[q];
+          T& ph = o.phi[q & 1][o.xx_of(1, q & 1, q >> 1)][q >> 1];
+          ph = ph + P.w6 * res[q];
         }
+      } else if (stall) {
+        o.template each<1>(lds, [&](int q, int yy, int xx, int zi, T r) {
+          if (ORDERED) res[q] = r;
+          sum[G::part(zi)] += fabs(r);
+          o.phi[yy][xx][zi] = o.phi[yy][xx][zi] + P.w6 * r;
+        });
+      } else {
+        o.template each<1>(lds, [&](int, int yy, int xx, int zi, T r) { o.phi[yy][xx][zi] = o.phi[yy][xx][zi] + P.w6 * r; });
       }
-    } else {
-      __syncthreads();
+      o.template publish<1>(lds);
+      blocks_sync<G>();
+      if (stall || (it + 1 >= first_check && (it + 1 - first_check) % P.check_every == 0)) {
+#pragma unroll
+        for (int h = 0; h < G::PARTS; h++) black_sum[h] = T(0);
+        o.template each<0>(lds, [&](int q, int yy, int xx, int zi, T r) {
+          if (ORDERED) black[q] = r;
+          black_sum[G::part(zi)] += fabs(r);
+          o.phi[yy][xx][zi] = o.phi[yy][xx][zi] + P.w6 * r;
+        });
+      } else {
+        o.template each<0>(lds, [&](int, int yy, int xx, int zi, T r) { o.phi[yy][xx][zi] = o.phi[yy][xx][zi] + P.w6 * r; });
+      }
+      o.template publish<0>(lds);
+      if (stall) {
+#pragma unroll
+        for (int h = 0; h < G::PARTS; h++) sum[h] = sum[h] + black_sum[h];
+        T tot = o.active ? tree_sum<G::PARTS>(sum) : T(0);
+        T* r2 = red + 2 * G::WAVES;
+        tot = wave_sum_dpp(tot);
+        blocks_put<G::WAVES>(tot, r2);
+        blocks_sync<G>();
+        tot = blocks_get<G::WAVES>(tot, r2);
+        if (it + 1 >= P.min_iter) {
+          bool grew = tot > old;
+          if constexpr (ORDERED) {
+            if (__builtin_expect(too_close(tot, old), 0) && (tot != old || blocks_moved<G::WAVES>(o, res, prev1, black, prev0, red))) {
+              float a = Ordered::column(o, res, lds);
+              a += Ordered::column(o, black, lds);
+              a = Ordered::wave(a, false, lds);
+              float b = FLT_MAX;
+              if (it > 0) {
+                b = Ordered::column(o, prev1, lds);
+                b += Ordered::column(o, prev0, lds);
+                b = Ordered::wave(b, false, lds);
+              }
+              grew = a > b;
+            }
+          }
+          if (grew) {
+            it_done = it + 1;
+            st = kStatusConverged;
+            break;
+          }
+        }
+        old = tot;
+        if (ORDERED) {
+#pragma unroll
+          for (int q = 0; q < 2 * H; q++) {
+            prev1[q] = res[q];
+            prev0[q] = black[q];
+          }
+        }
+      } else {
+        blocks_sync<G>();
+      }
     }
   }
 
@@ -686,7 +707,7 @@ constexpr int blocks_waves(int gs, bool f64, int planes) {
   return f64 ? (gs == 1 ? 4 : gs == 2 || gs == 4 ? 5 : 3) : planes == 4 ? 4 : gs == 1 ? 5 : 6;
 }
 
-template <int GS, int PLANES, typename PT, typename G = BlockGeo<GS, typename PT::real, PLANES>>
+template <int GS, int PLANES, typename PT, int HELP, typename G = BlockGeo<GS, typename PT::real, PLANES, HELP>>
 __global__ void __launch_bounds__(G::THREADS, blocks_waves(GS, G::F64, PLANES))
     sor_blocks_kernel(UniformBatchT<typename PT::real> b, PT P, int wave_dpp) {
   using T = typename PT::real;
@@ -695,7 +716,7 @@ __global__ void __launch_bounds__(G::THREADS, blocks_waves(GS, G::F64, PLANES))
   const int p = blockIdx.x;
   if (p >= b.npatch) return;
   const int W = gra_nxt(P.gra_ghost);
-  blocks_patch<GS, PLANES>(reinterpret_cast<T*>(blocks_smem), b.rho + (size_t)p * R3, b.cpot + (size_t)p * C3,
+  blocks_patch<GS, PLANES, HELP>(reinterpret_cast<T*>(blocks_smem), b.rho + (size_t)p * R3, b.cpot + (size_t)p * C3,
                            b.guess ? b.guess + (size_t)p * (P.init_mode == 3 ? N3 : R3) : nullptr,
                            b.pot_out + (size_t)p * W * W * W, b.flu ? b.flu + (size_t)p * kNComp * kPatchCells : nullptr,
                            b.iters ? b.iters + p : nullptr, b.status ? b.status + p : nullptr, P, wave_dpp != 0);
@@ -713,18 +734,18 @@ __global__ void __launch_bounds__(G::THREADS, blocks_waves(GS, false, PLANES))
   if (patch < 0 || patch >= b.npatch) return;
   const PatchDesc d = b.desc[patch];
   const int W = gra_nxt(P.gra_ghost);
-  blocks_patch<GS, PLANES>(reinterpret_cast<float*>(blocks_smem), b.rho + d.rho_off, b.cpot + d.cpot_off,
+  blocks_patch<GS, PLANES, 1>(reinterpret_cast<float*>(blocks_smem), b.rho + d.rho_off, b.cpot + d.cpot_off,
                            b.guess ? b.guess + d.rho_off : nullptr, b.pot_out + (size_t)patch * W * W * W,
                            b.flu ? b.flu + (size_t)patch * kNComp * kPatchCells : nullptr, b.iters ? b.iters + patch : nullptr,
                            b.status ? b.status + patch : nullptr, P, wave_dpp != 0);
 }
 
-template <int GS, int PLANES, typename PT>
+template <int GS, int PLANES, int HELP = 1, typename PT>
 hipError_t launch_as(const UniformBatchT<typename PT::real>& b, const PT& p, bool wave_dpp, hipStream_t s) {
   using T = typename PT::real;
-  using G = BlockGeo<GS, T, PLANES>;
+  using G = BlockGeo<GS, T, PLANES, HELP>;
   static_assert(sizeof(T) * G::WORDS <= 64 * 1024, "fits the default dynamic LDS limit");
-  hipLaunchKernelGGL((sor_blocks_kernel<GS, PLANES, PT>), dim3(b.npatch), dim3(G::THREADS), sizeof(T) * G::WORDS, s, b, p,
+  hipLaunchKernelGGL((sor_blocks_kernel<GS, PLANES, PT, HELP>), dim3(b.npatch), dim3(G::THREADS), sizeof(T) * G::WORDS, s, b, p,
                      wave_dpp ? 1 : 0);
   return hipGetLastError();
 }
@@ -744,12 +765,24 @@ hipError_t launch_tasks_as(const MixedBatch& b, const SolveParams& p, int ppw, i
 // 122 / 124, 256: 140 / 144, 512: 185 / 214, 4096: 1004 / 1250.
 bool two_planes(int gs, bool f64, int npatch) { return npatch <= (gs == 3 ? (f64 ? 512 : 1536) : (f64 ? 0 : 768)); }
 
+// Helpers at FP64 ghost size 1, where one wave owns a patch and would do its interpolation (four coarse cells per lane, one
+// after the other), window and gravity update by itself: 8 us beside the launch, where the iterations take 0.6 us each.  Three
+// more waves share those, and the owner needs no barriers.  MI355X, us per call without / with helpers, 8 patches: 10
+// iterations 19.9 / 13.4, 40: 37.7 / 29.7; 512: 22.4 / 16.3, 41.2 / 33.4; 1536 (six workgroups to a CU, one round): 32.5 /
+// 27.3, 52.9 / 47.5; 2048: 36.6 / 40.6, 58.4 / 75.4.  The 256-thread kernel before the block form: 8 patches 13.2, 33.8; 512:
+// 18.1, 44.5.
+constexpr int kHelpersTo = 1536;
+
 template <typename PT>
 hipError_t launch_blocks(const UniformBatchT<typename PT::real>& b, const PT& p, bool wave_dpp, hipStream_t s) {
   constexpr bool F64 = sizeof(typename PT::real) == 8;
   const bool two = two_planes(b.gs, F64, b.npatch);
   switch (b.gs) {
-    case 1: return launch_as<1, 2>(b, p, wave_dpp, s);
+    case 1:
+      if constexpr (F64) {
+        if (b.npatch <= kHelpersTo) return launch_as<1, 2, 4>(b, p, wave_dpp, s);
+      }
+      return launch_as<1, 2>(b, p, wave_dpp, s);
     case 2: return launch_as<2, 2>(b, p, wave_dpp, s);
     case 3: return two ? launch_as<3, 2>(b, p, wave_dpp, s) : launch_as<3, 4>(b, p, wave_dpp, s);
     case 4: return launch_as<4, 2>(b, p, wave_dpp, s);
