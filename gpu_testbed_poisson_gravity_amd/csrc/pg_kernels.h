@@ -134,8 +134,8 @@ struct ParamsByGs {
   SolveParams p[6];
 };
 
-// Per-ghost-size launch layout of the one-wavefront SOR kernel: patches per wavefront.  Chosen by the autotuner;
-// the default is the densest packing that fits one wavefront.
+// Per-ghost-size launch layout of the one-wavefront SOR kernel, and where the block form runs instead.  Chosen by the
+// autotuner or the caller; the default is the densest packing that fits one wavefront, and sor_blocks_limit.
 struct SorLayout {
   int blocks_to[6];        // largest batch that runs in the block form instead, by gs (0: none; set by the caller, by the
                            // autotuner, or sor_blocks_limit)
@@ -149,7 +149,8 @@ hipError_t launch_uniform(const UniformBatch& b, const SolveParams& p, const Sor
 hipError_t launch_gravity(const float* pot, float* flu, int npatch, int gra_ghost, float gra_const, int p5,
                           hipStream_t stream);
 // Persistent kernels of a mixed batch: SOR tasks (one wavefront each, gs 1/2 packed ppw1/ppw2 per
-// wavefront, default row padding) and MG tasks (one 256-thread workgroup per patch).
+// wavefront, default row padding) and MG tasks (one workgroup of 384
+// threads per patch, enough for any ghost size).
 hipError_t launch_sor_persistent(const MixedBatch& b, const ParamsByGs& p, int ppw1, int ppw2, int grid, size_t lds,
                                  hipStream_t stream);
 hipError_t launch_mg_persistent(const MixedBatch& b, const ParamsByGs& p, int grid, size_t lds, hipStream_t stream);

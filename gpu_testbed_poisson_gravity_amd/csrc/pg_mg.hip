@@ -56,7 +56,9 @@ constexpr MgLevels mg_levels_of(int n0) {
 // Dirichlet cells of that colour (y = 0, y = N-1, x = 0, x = N-1; MX each).  Where those and the planes start decides
 // the bank conflicts of the edge threads' reads and of waves that span two chunks of planes: the constants below were
 // found by search over the 32 lanes and 32 banks of an LDS cycle (GS 5: none left; with everything packed, half of
-// the LDS cycles of a V-cycle were conflicts, and LDS was the bound).
+// the LDS cycles of a V-cycle were conflicts, and LDS was the bound).  Searched: P, the faces' first words within P, and xs 1 or
+// MX, from random starts by single moves; counted: over all half waves and the seven addresses of a colour pass (own, ylo, yhi,
+// both xlo and both xhi), the most different words on one bank.
 // The cube's edges and corners, which no stencil reads, are not stored.  While the coarse levels run, the solution
 // is in registers only and the interior of this array holds the defect, rows of R in the same places.
 constexpr int kMgRows = 32;   // rows of 16 lanes in the largest workgroup

@@ -17,7 +17,9 @@
 // owned cell sits at a compile-time offset from one lane register (the cell across the x pair even at the cell's own word,
 // in the other colour), the Dirichlet layer included.  A cell update costs two LDS reads (across the x pair and the y
 // pair), one more at the ends of a chunk of planes, and one write.  HP and PL were chosen for the fewest bank conflicts of
-// 32 lanes per cycle (FP32) or 16 (FP64): none at ghost sizes 1 and 5.
+// 32 lanes per cycle (FP32) or 16 (FP64): none at ghost sizes 1 and 5.  (Tried: HP from N/2 to N/2 + 3, PL from N HP to N HP +
+// 16, both lane orders; counted: over the groups of lanes that share a cycle, the most different words on one bank among the
+// lanes' own words, which every other access is a constant away from.)
 // FP64 at ghost size 5 keeps a column's cells of one colour together instead, so that the two cells of a thread's column
 // are one 16-byte read or write (BlockGeo::PAIRS): 64 lanes in 4 cycles, as an 8-byte read.  It was bound by the LDS (70%
 // busy, VALU 64%); now the LDS is busy for half of the time and the VALU for 62%, and what is left is their latency with
@@ -705,8 +707,11 @@ __device__ __forceinline__ void blocks_patch(T* __restrict__ lds, const T* __res
   }
 }
 
-// Waves per SIMD the kernel is compiled for: FP64 as many as the patches that fit the LDS make, FP32 4 in 128 registers
-// (16 cells per thread) or 6 in 80 (8 cells).
+// Waves per SIMD the kernel is asked to be compiled for.  FP64, with what the registers then allow beside the LDS: GS 1, 4 (16
+// single waves of 17); GS 2, 5 (comes out at 76 registers, 6: more than the eleven workgroups of two waves); GS 3, 3 (two
+// planes 76 registers, six workgroups of four waves beside seven; four planes 130, six of two beside seven); GS 4, 5 (80, 6:
+// the four workgroups of six waves); GS 5, 3 (138, the three of four).  FP32 4 in 128 registers (16 cells per thread) or 6 in
+// 80 (8 cells), 5 at GS 1.
 constexpr int blocks_waves(int gs, bool f64, int planes) {
   return f64 ? (gs == 1 ? 4 : gs == 2 || gs == 4 ? 5 : 3) : planes == 4 ? 4 : gs == 1 ? 5 : 6;
 }
@@ -801,11 +806,17 @@ hipError_t launch_blocks(const UniformBatchT<typename PT::real>& b, const PT& p,
 
 }  // namespace
 
-// Largest batch for which the block form is the faster one.  MI355X, us per call, one wavefront per patch (or group) / blocks, FP32 to 1e-5
-// from the interpolated start: GS 1, 8 patches 84 / 40, 4096: 109 / 69, 16384: 252 / 248; GS 2, 8: 83 / 39, 16384: 471 / 406
-// (25 of 32 lanes against 125 of 128); GS 3, 8: 87 / 43, 2048: 129 / 102, 16384: 821 / 633 (36 of 64 lanes against 108 of
-// 128); GS 4, 8: 95 / 43, 1024: 121 / 92, 1280: 124 / 124, 1536: 132 / 146; GS 5, 8: 103 / 44, 1024: 136 / 95, 1280:
-// 141 / 136, 1536: 148 / 150 (the one-wavefront kernel needs fewer reductions and reads once a launch fills the GPU).
+// Largest batch for which the block form is the faster one.  MI355X, us per call, one wavefront per patch (or group) / blocks,
+// FP32, 10, 40 and 150 iterations with a test every 2:
+//   GS 1   256 patches 42/19 80/39 215/110   4096: 53/36 93/62 232/162   8192: 69/63 111/110 266/293   16384: 139/122 224/215 510/524
+//   GS 2   256: 32/14 76/37 239/120   4096: 52/42 114/112 331/357   5120: 79/48 184/131 554/409   16384: 188/127 405/357 1268/1155
+//   GS 3   1024: 37/23 91/60 280/190   2048: 45/35 110/90 332/276   16384: 313/230 761/575 2475/1944
+//   GS 4   1024: 40/27 100/80 320/260   1152: 43/35 106/107 333/359   1536: 45/43 111/132 340/453
+//   GS 5   1024: 47/32 113/84 358/258   1152: 51/43 122/119 377/389   1536: 54/46 128/126 379/410
+// GS 1 to 3: the one-wavefront kernel uses 25 of 32 lanes at GS 2 and 36 of 64 at GS 3.  It is ahead only where its waves just
+// fill a round and the solve is long (above some 60 iterations, 3700 to 4096 patches at GS 2, 7300 to 8192 and 16384 at GS 1).
+// GS 4 and 5: 1024 patches are four workgroups to a CU; beyond, long solves lose (the one-wavefront kernel needs fewer
+// reductions and reads once a launch fills the GPU).
 int sor_blocks_limit(int gs) { return gs <= 3 ? INT_MAX : 1024; }
 
 hipError_t launch_sor_blocks(const UniformBatch& b, const SolveParams& p, bool wave_dpp, hipStream_t s) {
