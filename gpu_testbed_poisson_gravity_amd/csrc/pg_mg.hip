@@ -898,12 +898,13 @@ __device__ void mg_patch_cells(T* __restrict__ lds, const T* __restrict__ rho, c
   }
 }
 
-// How a batch is run: mg_patch, or for a small batch at ghost sizes 1 and 2 mg_patch_cells (see mg_small).
-enum MgForm { kMgBlocks, kMgCells };
+// How a batch is run: mg_patch, or for a small batch at ghost sizes 1 and 2 mg_patch_cells (see mg_small), at ghost size 3
+// mg_patch with twice the threads (see mg_wide).
+enum MgForm { kMgBlocks, kMgCells, kMgWide };
 
 template <int GS, MgForm F, typename T>
 struct MgLaunch {
-  static constexpr int THREADS = F == kMgCells ? mg_cell_threads(GS) : MgGeo<GS>::THREADS;
+  static constexpr int THREADS = F == kMgCells ? mg_cell_threads(GS) : MgGeo<GS>::THREADS * (F == kMgWide ? 2 : 1);
   static constexpr int WAVES = F == kMgCells ? (sizeof(T) == 8 ? 2 : 6) : mg_waves(GS, sizeof(T));
   static constexpr size_t LDS = sizeof(T) * (MgGeo<GS>::FLOATS + (F == kMgCells ? MgGeo<GS>::N * MgGeo<GS>::N * MgGeo<GS>::N : 0));
 };
@@ -945,14 +946,22 @@ size_t lds_bytes_mg(int gs) {
   return 0;
 }
 
-// Largest batch for mg_patch_cells.  Measured on MI355X, us per call (interpolated start, 3+3 smoothing; FP32 to 1e-5,
-// FP64 to 1e-10), mg_patch / mg_patch_cells: FP32 GS 1, 512 patches 31 / 20, 1024: 32 / 26 (its limit: four workgroups
-// per CU), 1536: 38 / 37; GS 2, 256: 26 / 21, 512: 28.0 / 27.7 (two per CU), 1024: 31 / 43.  FP64 GS 1, 512: 64 / 52,
-// 1024: 71 / 101; GS 2, 256: 63 / 59 (one per CU), 512: 74 / 108.
+// Largest batch for mg_patch_cells.  Measured on MI355X, us per call (interpolated start, 3+3 smoothing), mg_patch /
+// mg_patch_cells after 1, 2 and 3 V-cycles (mg_patch's set-up is the longer, its V-cycle the shorter in a full GPU): FP32 GS 1,
+// 1025 patches 21.9/14.4 27.1/21.6 32.3/28.7, 1536: 24.4/17.8 29.7/26.5 35.4/34.6, 2048: 25.9/21.8 31.7/32.7 37.2/43.0; GS 2,
+// 513: 16.8/14.7 22.6/24.3 28.6/33.5 (two workgroups per CU to 512).  FP64, which goes on to six V-cycles for 1e-10: GS 1, 513:
+// 23.0/15.6 29.3/22.7 35.3/30.4, 768: 24.7/17.9 31.4/25.2 38.0/32.8, 1024: 26.6/25.9 33.0/36.9 39.2/47.9; GS 2, 257: 18.7/22.6
+// 26.3/35.4 33.9/48.1 (one per CU to 256).
 static bool mg_small(int gs, size_t word, int n) {
-  if (gs == 1) return n <= (word == 8 ? 512 : 1024);
+  if (gs == 1) return n <= (word == 8 ? 768 : 1536);
   return gs == 2 && n <= (word == 8 ? 256 : 512);
 }
+
+// Twice the threads for mg_patch at ghost size 3, one patch to a CU: the second half shares the interpolation, the window and
+// the gravity update.  us per call with 128 / 256 threads, 1, 3 and 6 V-cycles: FP32, 8 patches 20.0/17.5 38.9/36.9 67.5/65.8,
+// 256: 20.7/18.4 39.6/37.5 67.0/65.4, 320: 21.7/19.8 41.2/40.4 69.8/70.7; FP64, 8: 21.6/19.7 44.3/42.7 78.0/76.9, 256:
+// 22.9/21.3 44.9/44.4 76.9/76.5, 320: 27.1/25.3 53.6/53.9 92.2/94.4.
+static bool mg_wide(int gs, int n) { return gs == 3 && n <= 256; }
 
 template <int GS, MgForm F, typename PT>
 static hipError_t launch_mg_as(const UniformBatchT<typename PT::real>& b, const PT& p, hipStream_t s) {
@@ -968,6 +977,9 @@ template <int GS, typename PT>
 static hipError_t launch_mg(const UniformBatchT<typename PT::real>& b, const PT& p, hipStream_t s) {
   if constexpr (GS <= 2) {
     if (mg_small(GS, sizeof(typename PT::real), b.npatch)) return launch_mg_as<GS, kMgCells>(b, p, s);
+  }
+  if constexpr (GS == 3) {
+    if (mg_wide(GS, b.npatch)) return launch_mg_as<GS, kMgWide>(b, p, s);
   }
   return launch_mg_as<GS, kMgBlocks>(b, p, s);
 }
@@ -1030,6 +1042,9 @@ template <int GS>
 static void launch_mg_tasks_as(const MixedBatch& b, const SolveParams& p, int first, int count, hipStream_t s) {
   if constexpr (GS <= 2) {
     if (mg_small(GS, sizeof(float), count)) return launch_mg_tasks_form<GS, kMgCells>(b, p, first, count, s);
+  }
+  if constexpr (GS == 3) {
+    if (mg_wide(GS, count)) return launch_mg_tasks_form<GS, kMgWide>(b, p, first, count, s);
   }
   launch_mg_tasks_form<GS, kMgBlocks>(b, p, first, count, s);
 }

@@ -49,7 +49,7 @@ def _ms(ctx, batch):
 
 
 def _tune(ctx, batch):
-    return ctx.autotune(GS, batch[0], batch[1], batch[2], N, _args(), repeats=5)
+    return ctx.autotune(GS, batch[0], batch[1], batch[2], N, _args(), repeats=20)
 
 
 def test_putting_a_layout_back_restores_the_choice_of_form(batch):

@@ -67,3 +67,11 @@ def test_mg_whole_cube_window(gs):
     shell = np.ones(pot.shape[1:], bool)
     shell[1:-1, 1:-1, 1:-1] = False
     assert np.array_equal(pot[:, shell], cube[np.arange(n) % K][:, shell])
+
+
+@pytest.mark.parametrize("gs, n, dtype", [(1, 1536, np.float32), (1, 1537, np.float32), (1, 768, np.float64),
+                                          (1, 769, np.float64), (3, 256, np.float32), (3, 257, np.float32),
+                                          (3, 256, np.float64), (3, 257, np.float64)])
+def test_mg_forms_bitwise_at_their_limits(gs, n, dtype):
+    _check(gs, n, dtype)
+    _check(gs, n, dtype, gg=gs, graacc=False, smooth=(1, 0))

@@ -62,7 +62,9 @@ def _mg_error(rho, cube, dtype):
 
 
 @pytest.mark.parametrize("gs, sizes, dtype", [(1, (3, 1024, 1025), np.float32), (2, (3, 512, 513), np.float32),
-                                              (1, (3, 512, 513), np.float64), (2, (3, 256, 257), np.float64)])
+                                              (1, (3, 512, 513), np.float64), (2, (3, 256, 257), np.float64),
+                                              (1, (3, 1536, 1537), np.float32), (1, (3, 768, 769), np.float64),
+                                              (3, (3, 256, 257), np.float32), (3, (3, 256, 257), np.float64)])
 def test_mg_stops_alike_in_every_batch(gs, sizes, dtype):
     """Batch sizes on both sides of the line between one cell per thread and blocks of cells."""
     k = 3
