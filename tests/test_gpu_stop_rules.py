@@ -81,7 +81,7 @@ def test_mg_stops_alike_in_every_batch(gs, sizes, dtype):
     assert {1, 2, 3} <= counts
 
 
-@pytest.mark.parametrize("gs, sizes", [(1, (5, 1024, 1025)), (2, (5, 512, 513))])
+@pytest.mark.parametrize("gs, sizes", [(1, (5, 1025, 1536, 1537)), (2, (5, 512, 513)), (3, (5, 256, 257))])
 def test_mg_checks_guesses_alike_in_every_batch(gs, sizes):
     k, R, dtype = 5, 6 + 2 * gs, np.float32
     rho, cpot, _, _ = I.plummer(k, gs, seed=50 + gs)
@@ -108,7 +108,7 @@ def test_mg_slices_and_mixed_modes_stop_alike():
     """A host batch cut into slices against the same batch in one launch, and both modes of a mixed batch."""
     import torch
 
-    k, n, dtype = 3, 1032, np.float32   # slices of 512 and 520 patches, one launch of 1032
+    k, n, dtype = 3, 2056, np.float32   # slices of 1024, 512 and 520 patches, one launch of 2056
     at = np.arange(n) % k
     rho, cpot, _, _ = I.plummer(k, 1, seed=41)
     cube = _Solver(1, dtype, rho, cpot, k, pot_scheme=pg.MG, gra_ghost_size=1)(mg_max_iter=2, mg_tol=0.0)[0]
